@@ -384,3 +384,24 @@ def test_pooled_switch_above_the_decode_bound_takes_one_lru_pass(device):
         assert pool._free == ref.free, step
         assert hits >= 0
     assert ref.misses > 48                      # evictions happened
+
+
+@pytest.mark.parametrize("tokens", [12, 150, 330], ids=["16-row-class", "48-row-tiles", "96-row-tiles"])
+@pytest.mark.parametrize("inter", [384, 640, 896, 320], ids=["8+4", "8+8+4", "3x8+4", "8+2-clamped"])
+def test_down_gemm_half_chunk_tail(device, tokens, inter):
+    """Intermediate sizes of half a K chunk over (12, 20 and 28 groups) run
+    the down GEMM's staged half-tail instances, 10 groups the clamped tail.
+    One expert takes two thirds of the rows (several tiles, a ragged last
+    one); 330 tokens over 12 experts take the tall tiles.  Weight scales of
+    the last row end the bank, so a load past a row would be past its end."""
+    hidden, experts, k = 256, 12, 3
+    np_packs = packs(71, hidden, inter, experts)
+    rng = np.random.default_rng(72 + inter)
+    inds = np.stack([rng.choice(experts, k, replace=False) for _ in range(tokens)]).astype(np.int32)
+    inds[:2 * tokens // 3, 0] = experts - 1
+    x_np = mo.bf16r(rng.normal(size=(tokens, hidden)).astype(np.float32))
+    switch = _switch(np_packs, hidden, inter, experts, device)
+    out = grouped_experts(switch, bf16_device(x_np, device), torch.tensor(inds, device=device))
+    torch.cuda.synchronize()
+    _, _, _, d_out, _ = mo.execute(x_np, inds, np_packs, "bf16", qmm=True)
+    _close_qmm(host(out), d_out, f"inter {inter}, {tokens} rows")

@@ -559,7 +559,7 @@ static uint32_t gateup_tile_rows(uint32_t T, uint32_t K, uint32_t H, uint32_t E)
 // Rows per down tile: the same rule over the intermediate size and the down
 // GEMM's usual height (3072 rows 514-519 -> 502-508 us per call).
 static uint32_t down_tile_rows(uint32_t T, uint32_t K, uint32_t I, uint32_t E) {
-  const bool tall = uint64_t(T) * K > uint64_t(E) * vm::kGroupedRowsDown && I % (8 * 32) == 0;
+  const bool tall = uint64_t(T) * K > uint64_t(E) * vm::kGroupedRowsDown && vm::down_tall_supported(I);
   return tall ? vm::kGroupedRowsTall : vm::kGroupedRowsDown;
 }
 

@@ -97,6 +97,16 @@ __device__ __forceinline__ constexpr uint32_t w_swz(uint32_t c) { return c & 7u;
 #endif
 constexpr int kWColBytes = kCG * 16;  // LDS bytes per staged weight row chunk (unpadded: the groups are swizzled)
 
+// K of half a chunk over, after at least one whole chunk (K = 640: 8 + 8 + 4
+// groups; HALF instances): the last chunk is loaded from the row's last eight
+// groups, all of them inside the row, and only its upper half's MFMA steps
+// run, so rows, weights and scales are staged as in a whole chunk.  Any other
+// remainder (TAIL instances) has its last chunk's loads clamped and its lanes
+// fetch their own weights and 2-byte scales: at hidden 2560 / inter 640 those
+// took the 1999-row call 641 us where these take 596, and 333 rows 505 and
+// 449.  Same products in the same order: the same bits.
+constexpr bool half_tail(uint32_t groups) { return groups % kCG == kCG / 2 && groups > kCG; }
+
 // Q4 weights staged through LDS (coalesced 128-byte row loads by the whole
 // block) rather than loaded by the MFMA lanes themselves.
 template <int EPI, bool TAIL>
@@ -339,7 +349,7 @@ constexpr uint32_t slices_per_block() {
 // staging covers those rows only and the MFMA loops carry no branch, so the
 // LDS reads of a step and the MFMAs of neighbouring steps can be scheduled
 // freely.
-template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, int MBU, bool WNT, int TR>
+template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, int MBU, bool WNT, bool HALF, int TR>
 __device__ __forceinline__ void grouped_tile(const GroupedLaunch& p, const ProjPtrs (&w)[PROJ], uint32_t row0,
                                              uint32_t rows, uint32_t slice0, uint32_t nslices, uint8_t* s_a0) {
   constexpr bool Q4 = EPI != kEpiLogits;
@@ -534,7 +544,7 @@ __device__ __forceinline__ void grouped_tile(const GroupedLaunch& p, const ProjP
   // LDS-store phase instead, a higher level (2 or 3), or the same raise in the
   // down GEMM gained nothing consistent.
   constexpr bool kPrio = EPI == kEpiSwiglu;
-  auto compute = [&](int buf, const BChunk<Q4, TAIL> (&bc)[PROJ][NBW]) {
+  auto compute = [&](int buf, uint32_t c, const BChunk<Q4, TAIL> (&bc)[PROJ][NBW]) {
     if constexpr (kPrio) __builtin_amdgcn_s_setprio(1);
     const uint8_t* s_a = s_a0 + buf * kStage;
     BChunk<Q4, TAIL> bl[PROJ][NBW];
@@ -553,6 +563,8 @@ __device__ __forceinline__ void grouped_tile(const GroupedLaunch& p, const ProjP
       }
 #pragma unroll
     for (int st = 0; st < kSteps; ++st) {
+      // the last chunk of a half tail: the upper half only
+      if (HALF && st < kSteps / 2 && c + 1 == chunks) continue;
       const uint32_t a_step = (st >> 2) * 256u + (st & 3) * 16u;
       bf16x8_t aop[MBU];
 #pragma unroll
@@ -588,6 +600,9 @@ __device__ __forceinline__ void grouped_tile(const GroupedLaunch& p, const ProjP
   };
   // only a K that is not a multiple of the chunk has a tail chunk
   auto tail_chunk = [&](uint32_t c) { return TAIL && (c + 1) * kCG > G; };
+  // first group of chunk c (kTailHalf: the last chunk is the row's last eight
+  // groups, of which the upper four are new)
+  auto first_group = [&](uint32_t c) { return HALF ? min(c * kCG, G - kCG) : c * kCG; };
   // epilogue of slice s: lane holds rows 4*(lane/16) + i of every row block, column lane%16
   auto epilogue = [&](uint32_t s) {
 #pragma unroll
@@ -640,8 +655,8 @@ __device__ __forceinline__ void grouped_tile(const GroupedLaunch& p, const ProjP
       // one slice: the epilogue after the loop, where the loop's offsets are dead
       for (uint32_t c = 0; c < chunks; ++c) {
         const bool more = c + 1 < chunks;
-        if (more) a_load((c + 1) * kCG, tail_chunk(c + 1));
-        compute(0, b0);
+        if (more) a_load(first_group(c + 1), tail_chunk(c + 1));
+        compute(0, c, b0);
         __syncthreads();
         if (more) {
           a_store(0);
@@ -655,12 +670,12 @@ __device__ __forceinline__ void grouped_tile(const GroupedLaunch& p, const ProjP
       for (uint32_t c = 0; c < chunks; ++c) {
         const bool more = c + 1 < chunks || k + 1 < nslices;
         if (c + 1 < chunks) {
-          a_load((c + 1) * kCG, tail_chunk(c + 1));
+          a_load(first_group(c + 1), tail_chunk(c + 1));
         } else if (more) {
           next_slice();
           a_load(0, tail_chunk(0));
         }
-        compute(0, b0);
+        compute(0, c, b0);
         __syncthreads();
         if (more) {
           a_store(0);
@@ -687,10 +702,10 @@ __device__ __forceinline__ void grouped_tile(const GroupedLaunch& p, const ProjP
       const int buf = c & 1;
       const bool more = c + 1 < chunks;
       if (more) {
-        a_load((c + 1) * kCG, tail_chunk(c + 1));
-        b_load(b1, (c + 1) * kCG, tail_chunk(c + 1));
+        a_load(first_group(c + 1), tail_chunk(c + 1));
+        b_load(b1, first_group(c + 1), tail_chunk(c + 1));
       }
-      compute(buf, b0);
+      compute(buf, c, b0);
       if (more) {
         a_store(buf ^ 1);
 #pragma unroll
@@ -704,12 +719,13 @@ __device__ __forceinline__ void grouped_tile(const GroupedLaunch& p, const ProjP
   }
 }
 
-template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, bool WNT, int TR>
+template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, bool WNT, bool HALF, int TR>
 __device__ __forceinline__ void grouped_block(const GroupedLaunch& p, uint32_t lin, uint8_t* s_a0);
 
 // EPI: 0 SwiGLU of projections 0 (gate) and 1 (up) -> bf16 [rows, N];
 //      1 bf16 rows -> [rows, N]; 2 router logits (bf16 weights) -> fp32 [rows, N].
 // TAIL: K is not a multiple of the chunk (kCG groups); the last chunk clamps.
+// HALF: K has half a chunk over (see half_tail).
 #ifndef VM_G_WAVES_PER_EU
 #define VM_G_WAVES_PER_EU 1
 #endif
@@ -731,7 +747,7 @@ __device__ __forceinline__ void grouped_block(const GroupedLaunch& p, uint32_t l
 // 2048-row gate/up fetched 28 % above its bytes).  Calls with several row
 // tiles per expert keep cached loads (the tiles of an expert share its
 // weights in the L2; non-temporal loads there cost 5 %).
-template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, bool WNT, int TR>
+template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, bool WNT, bool HALF, int TR>
 __global__ __launch_bounds__(WAVES * 64)
 __attribute__((amdgpu_waves_per_eu(EPI == kEpiRows ? VM_DN_WAVES_PER_EU : VM_G_WAVES_PER_EU)))
 void k_grouped(GroupedLaunch p) {
@@ -752,11 +768,11 @@ void k_grouped(GroupedLaunch p) {
     if (blockIdx.x == 0 && p.zero_words != nullptr)
       for (uint32_t i = tid; i < p.zero_count; i += WAVES * 64) p.zero_words[i] = 0;
   }
-  grouped_block<EPI, WAVES, NBW, PROJ, TAIL, WNT, TR>(p, blockIdx.x, s_a0);
+  grouped_block<EPI, WAVES, NBW, PROJ, TAIL, WNT, HALF, TR>(p, blockIdx.x, s_a0);
 }
 
 // One block's work item `lin` (the XCD-aware order of k_grouped).
-template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, bool WNT, int TR>
+template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, bool WNT, bool HALF, int TR>
 __device__ __forceinline__ void grouped_block(const GroupedLaunch& p, uint32_t lin, uint8_t* s_a0) {
   constexpr int kBM = TR;
   constexpr int kMB = kBM / 16;  // MFMA row blocks
@@ -819,21 +835,21 @@ __device__ __forceinline__ void grouped_block(const GroupedLaunch& p, uint32_t l
   }
   const uint32_t mbu = (rows + 15) / 16;  // block-uniform, 1..kMB
   if constexpr (kMB >= 6) {
-    if (mbu >= 6) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 6, WNT, TR>(p, w, row0, rows, slice0, nslices, s_a0);
+    if (mbu >= 6) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 6, WNT, HALF, TR>(p, w, row0, rows, slice0, nslices, s_a0);
   }
   if constexpr (kMB >= 5) {
-    if (mbu >= 5) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 5, WNT, TR>(p, w, row0, rows, slice0, nslices, s_a0);
+    if (mbu >= 5) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 5, WNT, HALF, TR>(p, w, row0, rows, slice0, nslices, s_a0);
   }
   if constexpr (kMB >= 4) {
-    if (mbu >= 4) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 4, WNT, TR>(p, w, row0, rows, slice0, nslices, s_a0);
+    if (mbu >= 4) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 4, WNT, HALF, TR>(p, w, row0, rows, slice0, nslices, s_a0);
   }
   if constexpr (kMB >= 3) {
-    if (mbu >= 3) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 3, WNT, TR>(p, w, row0, rows, slice0, nslices, s_a0);
+    if (mbu >= 3) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 3, WNT, HALF, TR>(p, w, row0, rows, slice0, nslices, s_a0);
   }
   if constexpr (kMB >= 2) {
-    if (mbu >= 2) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 2, WNT, TR>(p, w, row0, rows, slice0, nslices, s_a0);
+    if (mbu >= 2) return grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 2, WNT, HALF, TR>(p, w, row0, rows, slice0, nslices, s_a0);
   }
-  grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 1, WNT, TR>(p, w, row0, rows, slice0, nslices, s_a0);
+  grouped_tile<EPI, WAVES, NBW, PROJ, TAIL, 1, WNT, HALF, TR>(p, w, row0, rows, slice0, nslices, s_a0);
 }
 
 // ------------------------------------------------------------- row tiles ---
@@ -1493,12 +1509,12 @@ hipError_t launch(const char* family, void (*kernel)(KArgs...), dim3 grid, dim3 
   return hipGetLastError();
 }
 
-template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, bool WNT, int TR = tile_rows<EPI>()>
+template <int EPI, int WAVES, int NBW, int PROJ, bool TAIL, bool WNT, bool HALF = false, int TR = tile_rows<EPI>()>
 hipError_t grouped_go_k(const char* family, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
   // one LDS stage with staged weights (see grouped_tile), else two
   constexpr uint32_t lds = (lds_weights<EPI, TAIL>() ? 1 : 2) * stage_bytes<EPI, WAVES, NBW, PROJ, TAIL, TR>();
   static_assert(lds <= 160u * 1024u, "the LDS of one block");
-  auto kernel = &k_grouped<EPI, WAVES, NBW, PROJ, TAIL, WNT, TR>;
+  auto kernel = &k_grouped<EPI, WAVES, NBW, PROJ, TAIL, WNT, HALF, TR>;
   static bool attr = false;  // one attribute call per kernel instance
   if (!attr) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1524,18 +1540,30 @@ hipError_t grouped_go_k(const char* family, const GroupedLaunch& p, uint32_t max
 
 template <int EPI, int WAVES, int NBW, int PROJ>
 hipError_t grouped_go(const char* family, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
+  const uint32_t groups = p.k_dim / kGroup;
+  const bool whole = groups % kCG == 0;
+  // the down GEMM has half-chunk instances (its K is the intermediate size)
+  const bool half = EPI == kEpiRows && half_tail(groups);
   if constexpr (EPI == kEpiSwiglu || EPI == kEpiRows) {
     // tall tiles: calls of many rows per group, whose groups then need fewer
-    // row tiles (each tile dequantises its expert's weights once); full
-    // chunks and cached weight loads only
+    // row tiles (each tile dequantises its expert's weights once); staged
+    // weights and cached weight loads only
     if (p.tile_rows == static_cast<uint32_t>(kGroupedRowsTall)) {
-      if ((p.k_dim / kGroup) % kCG != 0 || p.weights_once) return hipErrorInvalidValue;
-      return grouped_go_k<EPI, WAVES, NBW, PROJ, false, false, kGroupedRowsTall>(family, p, max_tiles, stream);
+      if ((!whole && !half) || p.weights_once) return hipErrorInvalidValue;
+      if constexpr (EPI == kEpiRows) {
+        if (half)
+          return grouped_go_k<EPI, WAVES, NBW, PROJ, false, false, true, kGroupedRowsTall>(family, p, max_tiles, stream);
+      }
+      return grouped_go_k<EPI, WAVES, NBW, PROJ, false, false, false, kGroupedRowsTall>(family, p, max_tiles, stream);
     }
   }
   if (p.tile_rows != 0 && p.tile_rows != static_cast<uint32_t>(tile_rows<EPI>())) return hipErrorInvalidValue;
-  if ((p.k_dim / kGroup) % kCG != 0)
-    return grouped_go_k<EPI, WAVES, NBW, PROJ, true, false>(family, p, max_tiles, stream);
+  if constexpr (EPI == kEpiRows) {
+    if (half && p.weights_once)
+      return grouped_go_k<EPI, WAVES, NBW, PROJ, false, true, true>(family, p, max_tiles, stream);
+    if (half) return grouped_go_k<EPI, WAVES, NBW, PROJ, false, false, true>(family, p, max_tiles, stream);
+  }
+  if (!whole) return grouped_go_k<EPI, WAVES, NBW, PROJ, true, false>(family, p, max_tiles, stream);
   if (lds_weights<EPI, false>() && p.weights_once)
     return grouped_go_k<EPI, WAVES, NBW, PROJ, false, lds_weights<EPI, false>()>(family, p, max_tiles, stream);
   return grouped_go_k<EPI, WAVES, NBW, PROJ, false, false>(family, p, max_tiles, stream);
@@ -1585,6 +1613,10 @@ hipError_t launch_grouped(int epi, const GroupedLaunch& p, uint32_t max_tiles, h
 // strides are compile-time; the A rows of a 16-row tile take 8 to 128 KiB of
 // LDS).  Other K take the chunked GEMM.
 constexpr uint32_t kRowsMaxK = 4096;
+
+bool down_tall_supported(uint32_t k_dim) {
+  return (k_dim / kGroup) % kCG == 0 || half_tail(k_dim / kGroup);
+}
 
 bool rows_supported(uint32_t k_dim) {
   return k_dim == 256 || k_dim == 512 || k_dim == 1024 || k_dim == 2048 || k_dim == kRowsMaxK;

@@ -305,6 +305,8 @@ hipError_t launch_grouped(int epi, const GroupedLaunch& p, uint32_t max_tiles, h
 // The 16-row tile kernels of small calls (see k_rows); false when K is above
 // their LDS bound.
 constexpr int kRowsTile = 16;
+// The down GEMM's staged-weight instances (and so its tall tiles) take this K.
+bool down_tall_supported(uint32_t k_dim);
 bool rows_supported(uint32_t k_dim);
 hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream);
 // Calls up to this many (token, slot) pairs sort in one block.
