@@ -109,13 +109,27 @@ __device__ __forceinline__ uint32_t ActF32::load_bits(const void* p, size_t i) {
 // MLX's stable sigmoid sequence, every step rounded to the activation type
 // (models/flashnext/metal_runtime.py:277-283), then silu(g) * u.
 
+// In bf16 (g is a bf16 value at every caller) the exponential is the hardware
+// exp2 of mag times the float above log2(e), and the reciprocal the hardware's,
+// scaled by 2^64 on both sides so that its subnormal results survive: a fifth
+// of the instructions of expf and the IEEE division, and the same bits for all
+// 65,536 inputs, NaN and infinities among them (with log2(e) rounded to
+// nearest one input differs).  The 8192-row layer call
+// (2048 / 512, ten of 512 experts) went from 1003 to 988 us with it, the
+// 2048-row call from 371.4 to 369.3.
 template <class A>
 __device__ __forceinline__ float sigmoid_act(float g) {
 #pragma clang fp contract(off)
   float mag = fabsf(g);
-  float e = A::round(expf(mag));
-  float den = A::round(1.0f + e);
-  float small = A::round(1.0f / den);
+  float small;
+  if constexpr (A::kBytes == 2) {
+    float e = A::round(__builtin_amdgcn_exp2f(mag * 0x1.715478p+0f));
+    float den = A::round(1.0f + e);
+    small = A::round(__builtin_amdgcn_rcpf(den * 0x1p-64f) * 0x1p-64f);
+  } else {
+    float den = 1.0f + expf(mag);
+    small = 1.0f / den;
+  }
   return g < 0.0f ? small : A::round(1.0f - small);
 }
 
