@@ -244,7 +244,7 @@ typedef struct VmLayerArgs {
  * a multiple of 64 dividing n, lowrank a multiple of 32 up to 256,
  * hc_count 1..VM_MAX_STREAMS, 16-byte aligned hidden rows.  The workspace
  * (vm_hyper_mix_workspace bytes) receives normed and d unless `normed` is
- * given. */
+ * given, and behind them scratch of larger bf16 calls. */
 typedef struct VmHyperArgs {
   const void* hidden;            /* [tokens, n] the residual streams */
   const void* norm_weight;       /* [n] hc_norm gain, activation dtype */
@@ -381,7 +381,8 @@ int vm_moe_layer_lru(const VmLayerArgs* args, const VmDeviceLru* lru, void* stre
 #define VM_STATIC_SCRATCH_BYTES (4ull << 20)
 int vm_moe_layer_static(const VmLayerArgs* args, void* stream);
 
-/* The hyper-connection before a branch (see VmHyperArgs): two launches. */
+/* The hyper-connection before a branch (see VmHyperArgs): two launches, three
+ * for larger bf16 calls. */
 uint64_t vm_hyper_mix_workspace(uint32_t tokens, uint32_t hc_count, uint32_t hidden_size, uint32_t lowrank,
                                 uint32_t act_dtype);
 int vm_hyper_mix(const VmHyperArgs* args, void* stream);

@@ -72,6 +72,38 @@ def test_hyper_mix_matches_the_oracle(device, hc, H, r, T, group):
     assert_close(host(mixed), want_m, f"mixed T={T}")
 
 
+@pytest.mark.parametrize("hc,H,r,T,group,one_centered", [
+    (4, 2560, 32, 67, 0, True), (4, 256, 32, 641, 256, False), (2, 512, 64, 655, 0, True), (5, 512, 32, 257, 512, True),
+    (4, 2048, 96, 80, 0, True), (1, 4096, 32, 160, 64, True)])
+def test_hyper_mix_tiles_match_the_oracle_and_the_per_token_kernels(device, hc, H, r, T, group, one_centered):
+    """Calls of 655,360 stream values and more: 16-token tiles with a ragged last one, more than 48 projection
+    rows, several norm groups, every stream-count instance.  The per-token kernels serve the same call from a
+    workspace without the tiles' scratch: the normalised streams are the same bits."""
+    rng = np.random.default_rng(SEED + H + T)
+    parts = _hyper_np(rng, hc, H, r)
+    x, xd = _streams(rng, T, hc * H, device)
+    hyper = _hyper_dev(parts, hc, device, norm_group=group, one_centered=one_centered)
+    mixed, _, weights = hyper(xd)
+    n = hc * H
+    normed_bytes = (2 * T * n + 255) // 256 * 256
+    base = normed_bytes + (2 * T * r + 255) // 256 * 256
+    ws = hyper._ws[(T, 0, xd.device)]
+    assert ws.numel() > base
+    normed = ws[: 2 * T * n].clone()
+    low = ws[normed_bytes: normed_bytes + 2 * T * r].clone().view(torch.bfloat16)
+    hyper._ws[(T, 0, xd.device)] = torch.zeros(base, dtype=torch.uint8, device=device)
+    mixed1, _, weights1 = hyper(xd)
+    torch.cuda.synchronize()
+    one = hyper._ws[(T, 0, xd.device)]
+    assert torch.equal(one[: 2 * T * n], normed)
+    low1 = one[normed_bytes: normed_bytes + 2 * T * r].view(torch.bfloat16)
+    for got, per_token, what in ((low, low1, "d"), (weights, weights1, "weights"), (mixed, mixed1, "mixed")):
+        assert_close(host(got).reshape(T, -1), host(per_token).reshape(T, -1), f"{what}: tiles and per token")
+    want_m, want_w, _ = go.hyper_mix(x, *parts, hc, 1e-6, group_size=group, one_centered=one_centered)
+    assert_close(host(weights), want_w, f"weights T={T}")
+    assert_close(host(mixed), want_m, f"mixed T={T}")
+
+
 def test_hyper_mix_float32(device):
     hc, H, r, T = 4, 256, 32, 2
     rng = np.random.default_rng(SEED)

@@ -889,15 +889,26 @@ static int host_device_pointer(const void* host, const uint8_t** out) {
   return VM_OK;
 }
 
-// Workspace of vm_hyper_mix: normed [T, n] then d [T, lowrank], activation dtype.
+// Workspace of vm_hyper_mix: normed [T, n] then d [T, lowrank], activation
+// dtype, then the scratch of 16-token tiles (a call with less room than that
+// runs the per-token kernels).
 static uint64_t hyper_normed_bytes(uint32_t tokens, uint32_t n, uint32_t act_dtype) {
   return align_up(uint64_t(tokens) * n * (act_dtype == VM_F32 ? 4 : 2));
+}
+
+static uint64_t hyper_base_bytes(uint32_t tokens, uint32_t n, uint32_t lowrank, uint32_t act_dtype) {
+  return hyper_normed_bytes(tokens, n, act_dtype) + align_up(uint64_t(tokens) * lowrank * (act_dtype == VM_F32 ? 4 : 2));
+}
+
+static uint64_t hyper_scratch_bytes(uint32_t tokens, uint32_t n, uint32_t rows, uint32_t act_dtype) {
+  return act_dtype == VM_BF16 && uint64_t(tokens) * n >= vm::kHcTileMin ? align_up(vm::hyper_tile_bytes(tokens, n, rows)) : 0;
 }
 
 uint64_t vm_hyper_mix_workspace(uint32_t tokens, uint32_t hc_count, uint32_t hidden_size, uint32_t lowrank,
                                 uint32_t act_dtype) {
   const uint32_t n = hc_count * hidden_size;
-  return hyper_normed_bytes(tokens, n, act_dtype) + align_up(uint64_t(tokens) * lowrank * (act_dtype == VM_F32 ? 4 : 2));
+  return hyper_base_bytes(tokens, n, lowrank, act_dtype) +
+         hyper_scratch_bytes(tokens, n, lowrank + hc_count, act_dtype);
 }
 
 int vm_hyper_mix(const VmHyperArgs* a, void* stream_ptr) {
@@ -923,11 +934,14 @@ int vm_hyper_mix(const VmHyperArgs* a, void* stream_ptr) {
     return fail(VM_EINVAL, "mix_down, mix_up and inject projections are required");
   if (!aligned16(a->mix_down.weight) || !aligned16(a->mix_up.weight) || !aligned16(a->inject.weight))
     return fail(VM_EINVAL, "projection weights must be 16-byte aligned");
-  const uint64_t need = vm_hyper_mix_workspace(T, hc, H, r, a->act_dtype);
+  const uint64_t need = hyper_base_bytes(T, n, r, a->act_dtype);
   if (a->workspace == nullptr || a->workspace_bytes < need)
     return fail(VM_EWORKSPACE, "workspace of %llu bytes needed", (unsigned long long)need);
   char* ws = static_cast<char*>(a->workspace);
+  const uint64_t scratch = hyper_scratch_bytes(T, n, r + hc, a->act_dtype);
   vm::HcLaunch p{};
+  if (scratch != 0 && a->workspace_bytes >= need + scratch && aligned16(ws))
+    p.tile_ws = reinterpret_cast<float*>(ws + need);
   p.hidden = a->hidden;
   p.norm_weight = a->norm_weight;
   p.down = to_ptrs(a->mix_down);

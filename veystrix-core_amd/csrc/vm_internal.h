@@ -368,10 +368,23 @@ struct HcLaunch {
   void* d;                     // [T, lowrank]
   void* mixed;                 // [T, hidden]
   void* weights;               // [T, hc]
+  float* tile_ws;              // hyper_tile_bytes of scratch, or null (no 16-token tiles)
   float eps;
   uint32_t tokens, width, hc, n, lowrank, norm_group, one_centered;  // width = hidden size
   int act_dtype;
 };
+
+// bf16 calls of at least this many stream values (tokens * n) run 16-token
+// tiles (glue.hip) when hyper_tiled accepts the call.  Below it the three tile
+// kernels are a chain of latencies: n = 10240, 48 / 64 / 128 tokens 18.4 / 18.5
+// / 19.4 us against 14.4 / 19.5 / 28.4 us per token; n = 4096, 128 / 256 tokens
+// 18.3 / 18.9 against 17.3 / 27.7.  hyper_tile_bytes is the scratch they need
+// beside normed and d, for `rows` = lowrank + hc projection rows.
+#ifndef VM_HC_TILE_MIN
+#define VM_HC_TILE_MIN (640 * 1024)
+#endif
+constexpr uint64_t kHcTileMin = VM_HC_TILE_MIN;
+uint64_t hyper_tile_bytes(uint32_t tokens, uint32_t n, uint32_t rows);
 
 hipError_t launch_hyper_mix(const HcLaunch& p, hipStream_t stream);
 
