@@ -84,6 +84,18 @@ def test_decode_small_layer_fp32(device):
     _check_layer(layer, spec, 7, x_np, "f32", device)
 
 
+@pytest.mark.parametrize("hidden,inter", [(2560, 96), (1280, 640), (640, 320), (320, 1280), (256, 640)])
+@pytest.mark.parametrize("tokens,mode", [(1, "bf16"), (5, "bf16"), (3, "f32")])
+def test_decode_rows_a_quarter_over_a_power_of_two(device, hidden, inter, tokens, mode):
+    """Rows of 10, 20, 40 and 80 groups, whose last quarters share loads, in gate/up and down; the shared expert of
+    the same widths, an output tile that ends inside a block (inter 96)."""
+    spec = synth.LayerSpec("quarter", hidden, inter, 16, 4, inter, tokens)
+    seed = hidden + inter
+    layer = assemble.build_layer(spec, seed, device, dense=True)
+    x_np = mo.bf16_bits_to_f32(synth.tokens(spec, seed, tokens))
+    _check_layer(layer, spec, seed, x_np, mode, device)
+
+
 @pytest.fixture(scope="module")
 def full_layer(device):
     spec = synth.CONFIGS["decode"]

@@ -56,11 +56,11 @@ constexpr int kFrontW = VM_FRONT_WAVES;
 #define VM_DOWN_QUADS 2
 #endif
 constexpr int kGateupRowsPerLane = VM_GATEUP_ROWS;
-#ifndef VM_GATEUP_WAVES
-#define VM_GATEUP_WAVES 2
-#endif
-constexpr int kGuWaves = VM_GATEUP_WAVES;  // waves per gate/up block
-constexpr int kGuBlock = kGuWaves * 64;
+// waves per gate/up block: two for one token, whose few blocks are spread over
+// more CUs so; four for more tokens, where half as many blocks repeat the
+// selection (hidden 2048: 2 / 5 / 8 tokens 20.7 / 39.4 / 53.7 us per layer with
+// two, 20.0 / 38.5 / 52.8 with four; hidden 2560 the same within 1 %)
+constexpr int kGuWaves = 2, kGuWavesMulti = 4;
 template <class A, bool GATE = false>
 __device__ void select_body(const SelectLaunch& p) {
   __shared__ typename Cand<A>::T s_cand[kMaxCand];
@@ -182,19 +182,25 @@ __device__ __forceinline__ void gateup_store(const GateUpLaunch& p, uint32_t t, 
 }
 
 // LPR lanes per row (one 32-input group per lane and iteration, GI
-// iterations), U rows per lane group; a block covers RPB = (64/LPR)*U*4 rows.
-template <class A, int LPR, int GI, int U>
-__global__ __launch_bounds__(kGuBlock) void k_gateup(GateUpLaunch p) {
+// iterations), U rows per lane group; a block covers RPB = (64/LPR)*U*WAVES rows.
+// FOLD: rows of LPR (1 + 1 / FOLD) groups; the groups over of FOLD rows share
+// one load of the whole lane group (quarter_over), GI is 1.
+template <class A, int LPR, int GI, int U, int FOLD, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void k_gateup(GateUpLaunch p) {
   constexpr int RPI = 64 / LPR;
   constexpr int RPW = RPI * U;
-  constexpr int RPB = RPW * kGuWaves;
+  constexpr int RPB = RPW * WAVES;
+  constexpr int NX = GI + (FOLD ? 1 : 0);              // activation groups per lane
+  constexpr int NF = FOLD ? (U + FOLD - 1) / FOLD : 0;  // folded loads per lane and projection
+  constexpr int REM = FOLD ? LPR / FOLD : 1;            // groups over of a row
+  static_assert(FOLD == 0 || GI == 1, "folded rows have one whole group per lane");
   // every wave runs the selection itself (its own candidate list), so no
   // barrier stands between the selection and the weight loads
-  __shared__ typename Cand<A>::T s_cands[kGuWaves][kMaxCand];
+  __shared__ typename Cand<A>::T s_cands[WAVES][kMaxCand];
 
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
-  const uint32_t wave = tid >> 6;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   typename Cand<A>::T* s_cand = s_cands[wave];
   const uint32_t lr = lane % LPR;
   const uint32_t rw = lane / LPR;
@@ -237,11 +243,11 @@ __global__ __launch_bounds__(kGuBlock) void k_gateup(GateUpLaunch p) {
     }
   }
   asm volatile("" ::: "memory");
-  GroupAct<A> xa[GI];
+  GroupAct<A> xa[NX];
 #pragma unroll
-  for (int it = 0; it < GI; ++it) {
-    const uint32_t g = lr + it * LPR;
-    const bool live = g < G;
+  for (int it = 0; it < NX; ++it) {
+    const uint32_t g = it * LPR + (it == GI ? lr % REM : lr);
+    const bool live = FOLD || g < G;
     xa[it].fetch(live ? p.x : g_zero_page, live ? static_cast<size_t>(t) * H + g * kGroup : 0);
   }
 
@@ -266,7 +272,7 @@ __global__ __launch_bounds__(kGuBlock) void k_gateup(GateUpLaunch p) {
       if (p.trace != nullptr) tr.mark(6);
     }
     lds_barrier();
-    word = s_word;
+    word = __builtin_amdgcn_readfirstlane(s_word);
   } else if (!shared_pair) {
     word = p.routes[t * p.slots + j];
   }
@@ -287,29 +293,46 @@ __global__ __launch_bounds__(kGuBlock) void k_gateup(GateUpLaunch p) {
   if (!ok && tid == 0 && blockIdx.x == 0) flag(p.status, 1u);
   if (p.trace != nullptr) tr.mark(1);
 
-  // 3. stream the gate and up rows
+  // 3. stream the gate and up rows: scalar bases and 32-bit offsets.  Rows past
+  //    the end repeat the last one (not stored), lanes past the row's groups its
+  //    last group with scale and bias 0, an unresolved route the zero page.
   const uint32_t row_base = blockIdx.x * RPB + wave * RPW + rw;
-  const uint32_t* zw = reinterpret_cast<const uint32_t*>(g_zero_page) + lr * kWordsPerGroup;
-  const uint16_t* zm = reinterpret_cast<const uint16_t*>(g_zero_page) + lr;
+  const uint32_t okm = ok ? ~0u : 0u;
+  const auto base = [&](const void* q) { return static_cast<const uint8_t*>(ok ? q : g_zero_page); };
+  const uint8_t* gw = base(gp.w);
+  const uint8_t* gsc = base(gp.s);
+  const uint8_t* gbi = base(gp.b);
+  const uint8_t* uw = base(upp.w);
+  const uint8_t* usc = base(upp.s);
+  const uint8_t* ubi = base(upp.b);
   uint4 wg[U][GI], wu[U][GI];
   uint32_t sg[U][GI], bg[U][GI], su[U][GI], bu[U][GI];
-  const size_t row_words = H / 8;
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    const uint32_t row = row_base + u * RPI;
 #pragma unroll
     for (int it = 0; it < GI; ++it) {
       const uint32_t g = lr + it * LPR;
-      const bool live = ok && row < I && g < G;
-      const size_t wo = static_cast<size_t>(row) * row_words + g * kWordsPerGroup;
-      const size_t mo = static_cast<size_t>(row) * G + g;
-      wg[u][it] = ldg16(live ? gp.w + wo : zw);
-      wu[u][it] = ldg16(live ? upp.w + wo : zw);
-      sg[u][it] = ldg_u16(live ? gp.s + mo : zm);
-      bg[u][it] = ldg_u16(live ? gp.b + mo : zm);
-      su[u][it] = ldg_u16(live ? upp.s + mo : zm);
-      bu[u][it] = ldg_u16(live ? upp.b + mo : zm);
+      const uint32_t at = (min(row_base + u * RPI, I - 1) * G + (FOLD ? g : min(g, G - 1))) & okm;
+      wg[u][it] = ldg16(gw + at * 16u);
+      wu[u][it] = ldg16(uw + at * 16u);
+      sg[u][it] = ldg_u16(gsc + at * 2u);
+      bg[u][it] = ldg_u16(gbi + at * 2u);
+      su[u][it] = ldg_u16(usc + at * 2u);
+      bu[u][it] = ldg_u16(ubi + at * 2u);
     }
+  }
+  uint4 fg[NF + !NF], fu[NF + !NF];
+  uint32_t fsg[NF + !NF], fbg[NF + !NF], fsu[NF + !NF], fbu[NF + !NF];
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const uint32_t u = min(f * FOLD + lr / REM, static_cast<uint32_t>(U - 1));  // lanes past U: not used
+    const uint32_t at = (min(row_base + u * RPI, I - 1) * G + LPR + lr % REM) & okm;
+    fg[f] = ldg16(gw + at * 16u);
+    fu[f] = ldg16(uw + at * 16u);
+    fsg[f] = ldg_u16(gsc + at * 2u);
+    fbg[f] = ldg_u16(gbi + at * 2u);
+    fsu[f] = ldg_u16(usc + at * 2u);
+    fbu[f] = ldg_u16(ubi + at * 2u);
   }
 
   // 4. one block per token publishes the ordered selection for the down kernel
@@ -327,15 +350,27 @@ __global__ __launch_bounds__(kGuBlock) void k_gateup(GateUpLaunch p) {
 
   // 5. group dots, row sums, SwiGLU
 #pragma unroll
-  for (int it = 0; it < GI; ++it) xa[it].prepare();
+  for (int it = 0; it < NX; ++it) xa[it].prepare();
   float gs[U], us[U];
+  float over_g[NF + !NF], over_u[NF + !NF];  // the folded groups: lane part u % FOLD belongs to row u
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    over_g[f] = xa[NX - 1].apply(fg[f], bf16_to_f32(fsg[f]), bf16_to_f32(fbg[f]));
+    over_u[f] = xa[NX - 1].apply(fu[f], bf16_to_f32(fsu[f]), bf16_to_f32(fbu[f]));
+  }
 #pragma unroll
   for (int u = 0; u < U; ++u) {
     float ag = 0.0f, au = 0.0f;
 #pragma unroll
     for (int it = 0; it < GI; ++it) {
-      ag += xa[it].apply(wg[u][it], bf16_to_f32(sg[u][it]), bf16_to_f32(bg[u][it]));
-      au += xa[it].apply(wu[u][it], bf16_to_f32(su[u][it]), bf16_to_f32(bu[u][it]));
+      const uint32_t has = FOLD || lr + it * LPR < G ? ~0u : 0u;
+      ag += xa[it].apply(wg[u][it], bf16_to_f32(sg[u][it] & has), bf16_to_f32(bg[u][it] & has));
+      au += xa[it].apply(wu[u][it], bf16_to_f32(su[u][it] & has), bf16_to_f32(bu[u][it] & has));
+    }
+    if constexpr (FOLD > 0) {
+      const bool mine = lr / REM == static_cast<uint32_t>(u % FOLD);
+      ag += mine ? over_g[u / FOLD] : 0.0f;
+      au += mine ? over_u[u / FOLD] : 0.0f;
     }
     gs[u] = group_sum<LPR>(ag);
     us[u] = group_sum<LPR>(au);
@@ -382,10 +417,14 @@ constexpr int kDownQuads = VM_DOWN_QUADS;                 // row groups of 64/LP
 // slots of one token.
 // INJ: the combined rows are also injected into residual streams (p.inject);
 // a separate instance, so the plain kernel carries none of its loads.
-template <class A, int LPR, bool INJ>
+// FOLD: rows of LPR (1 + 1 / FOLD) groups (quarter_over).
+template <class A, int LPR, bool INJ, int FOLD, int QUADS>
 __global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
   constexpr int RPI = 64 / LPR;
-  constexpr int RB = RPI * kDownQuads;
+  constexpr int RB = RPI * QUADS;
+  constexpr int NX = FOLD ? 2 : 1;                          // activation groups per lane and slot
+  constexpr int NF = FOLD ? (QUADS + FOLD - 1) / FOLD : 0;  // folded loads per lane and slot
+  constexpr int REM = FOLD ? LPR / FOLD : 1;                // groups over of a row
   __shared__ float s_part[kDownMaxSlots * RB];
   __shared__ float s_scores[kDownMaxSlots];
   __shared__ float s_shared[RB];
@@ -393,7 +432,7 @@ __global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
 
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
-  const uint32_t wave = tid >> 6;
+  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const uint32_t lr = lane % LPR;
   const uint32_t rw = lane / LPR;
   const uint32_t t = blockIdx.y;
@@ -417,31 +456,32 @@ __global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
   //    wave's activation groups (slot wave + 4 i, group lr)
   const uint32_t route = ldg_u32(p.routes + static_cast<size_t>(t) * K + min(lane, K - 1));
   asm volatile("" ::: "memory");
-  GroupAct<A> xa[kDownSlotsPerWave];
+  GroupAct<A> xa[kDownSlotsPerWave][NX];
 #pragma unroll
   for (int i = 0; i < kDownSlotsPerWave; ++i) {
     const uint32_t slot = wave + kDownWaves * i;
-    const bool live = slot < S && lr < G;
-    xa[i].fetch(live ? p.act : g_zero_page, live ? (static_cast<size_t>(t) * S + slot) * I + lr * kGroup : 0);
+#pragma unroll
+    for (int x = 0; x < NX; ++x) {
+      const uint32_t g = x ? LPR + lr % REM : lr;
+      const bool live = slot < S && g < G;
+      xa[i][x].fetch(live ? p.act : g_zero_page, live ? (static_cast<size_t>(t) * S + slot) * I + g * kGroup : 0);
+    }
   }
 
-  // epilogue operands as raw bits: loaded now, converted into LDS after the
-  // weight loads are issued, so no load waits in front of those
+  // epilogue operands into LDS, by the last wave: with up to eleven slots it has
+  // no weights, so no register of the other waves holds them and no load waits
+  // in front of the weight loads
   const bool combine = p.scores != nullptr;
-  const uint32_t er = tid - 64;  // wave 1 fetches the shared term of the tile
   const void* sh_src = p.shared_y != nullptr ? p.shared_y : p.shared;
-  const bool take_score = combine && tid < K;
-  const bool take_shared = combine && tid >= 64 && er < RB && row0 + er < H && sh_src != nullptr;
   const void* sig_src = p.has_shared ? p.shared_sig : p.shared != nullptr ? p.shared_gate : nullptr;
-  const bool take_sig = combine && tid == 128 && sig_src != nullptr;
-  uint32_t r_score = 0, r_shared = 0, r_sig = 0;
-  if (take_score) {
-    const size_t o = static_cast<size_t>(t) * K + tid;
-    r_score = p.score_dtype == 0 ? ldg_u16(static_cast<const uint16_t*>(p.scores) + o)
-                                 : ldg_u32(static_cast<const uint32_t*>(p.scores) + o);
+  if (combine && wave == kDownWaves - 1) {
+    if (lane < K) s_scores[lane] = load_any(p.scores, static_cast<size_t>(t) * K + lane, p.score_dtype);
+    if (sh_src != nullptr) {
+      for (uint32_t r = lane; r < RB; r += 64)
+        if (row0 + r < H) s_shared[r] = A::load(sh_src, static_cast<size_t>(t) * H + row0 + r);
+    }
+    if (lane == 0 && sig_src != nullptr) s_sig = A::load(sig_src, t);
   }
-  if (take_shared) r_shared = A::load_bits(sh_src, static_cast<size_t>(t) * H + row0 + er);
-  if (take_sig) r_sig = A::load_bits(sig_src, t);
   // the streams this thread's combined row is injected into, and their weights
   const Inject& inj = p.inject;
   const bool take_inject = INJ && combine && tid < RB && row0 + tid < H;
@@ -467,11 +507,9 @@ __global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
   if (!mine_ok && lane < K && wave == 0 && blockIdx.x == 0) flag(p.status, 1u);
   const uint64_t ok_mask = __ballot(mine_ok);
   if (p.trace != nullptr) tr.mark(5);
-  const uint32_t* zw = reinterpret_cast<const uint32_t*>(g_zero_page) + lr * kWordsPerGroup;
-  const uint16_t* zm = reinterpret_cast<const uint16_t*>(g_zero_page) + lr;
-  uint4 w[kDownSlotsPerWave][kDownQuads];
-  uint32_t sc[kDownSlotsPerWave][kDownQuads], bi[kDownSlotsPerWave][kDownQuads];
-  const size_t row_words = I / 8;
+  constexpr int NL = QUADS + NF;  // loads per lane and slot, the folded ones last
+  uint4 w[kDownSlotsPerWave][NL];
+  uint32_t sc[kDownSlotsPerWave][NL], bi[kDownSlotsPerWave][NL];
 #pragma unroll
   for (int i = 0; i < kDownSlotsPerWave; ++i) {
     // no branch around the loads: slots past S load zeros, so the first use
@@ -485,33 +523,42 @@ __global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
       dp.s = reinterpret_cast<const uint16_t*>(readlane_u64(reinterpret_cast<uint64_t>(mine.s), slot));
       dp.b = reinterpret_cast<const uint16_t*>(readlane_u64(reinterpret_cast<uint64_t>(mine.b), slot));
     }
+    const uint32_t okm = ok ? ~0u : 0u;
+    const uint8_t* bw = static_cast<const uint8_t*>(ok ? static_cast<const void*>(dp.w) : g_zero_page);
+    const uint8_t* bs = static_cast<const uint8_t*>(ok ? static_cast<const void*>(dp.s) : g_zero_page);
+    const uint8_t* bb = static_cast<const uint8_t*>(ok ? static_cast<const void*>(dp.b) : g_zero_page);
 #pragma unroll
-    for (int q = 0; q < kDownQuads; ++q) {
-      const uint32_t row = row0 + q * RPI + rw;
-      const bool live = ok && row < H && lr < G;
-      const size_t mo = static_cast<size_t>(row) * G + lr;
-      w[i][q] = ldg16(live ? dp.w + static_cast<size_t>(row) * row_words + lr * kWordsPerGroup : zw);
-      sc[i][q] = ldg_u16(live ? dp.s + mo : zm);
-      bi[i][q] = ldg_u16(live ? dp.b + mo : zm);
+    for (int q = 0; q < NL; ++q) {
+      // rows past the end repeat the last one, lanes past the row's groups its
+      // last group with scale and bias 0
+      const bool folded = q >= QUADS;
+      const uint32_t qr = folded ? min((q - QUADS) * FOLD + lr / REM, static_cast<uint32_t>(QUADS - 1)) : q;
+      const uint32_t g = folded ? LPR + lr % REM : FOLD ? lr : min(lr, G - 1);
+      const uint32_t at = (min(row0 + qr * RPI + rw, H - 1) * G + g) & okm;
+      w[i][q] = ldg16(bw + at * 16u);
+      sc[i][q] = ldg_u16(bs + at * 2u);
+      bi[i][q] = ldg_u16(bb + at * 2u);
     }
   }
   if (p.trace != nullptr) tr.mark(6);
-
-  // 3. epilogue operands into LDS
-  if (take_score) s_scores[tid] = p.score_dtype == 0 ? bf16_to_f32(r_score) : __uint_as_float(r_score);
-  if (take_shared) s_shared[er] = A::from_bits(r_shared);
-  if (take_sig) s_sig = A::from_bits(r_sig);
   if (p.trace != nullptr) tr.mark(7);
 
-  // 4. dot products and row sums into LDS
+  // 3. dot products and row sums into LDS
 #pragma unroll
   for (int i = 0; i < kDownSlotsPerWave; ++i) {
     const uint32_t slot = wave + kDownWaves * i;
     if (slot >= S) break;  // wave-uniform
-    xa[i].prepare();
 #pragma unroll
-    for (int q = 0; q < kDownQuads; ++q) {
-      float v = xa[i].apply(w[i][q], bf16_to_f32(sc[i][q]), bf16_to_f32(bi[i][q]));
+    for (int x = 0; x < NX; ++x) xa[i][x].prepare();
+    float over[NF + !NF];
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      over[f] = xa[i][NX - 1].apply(w[i][QUADS + f], bf16_to_f32(sc[i][QUADS + f]), bf16_to_f32(bi[i][QUADS + f]));
+#pragma unroll
+    for (int q = 0; q < QUADS; ++q) {
+      const uint32_t has = FOLD || lr < G ? ~0u : 0u;
+      float v = xa[i][0].apply(w[i][q], bf16_to_f32(sc[i][q] & has), bf16_to_f32(bi[i][q] & has));
+      if constexpr (FOLD > 0) v += lr / REM == static_cast<uint32_t>(q % FOLD) ? over[q / FOLD] : 0.0f;
       v = group_sum<LPR>(v);
       if (lr == LPR - 1) s_part[slot * RB + q * RPI + rw] = v;
     }
@@ -521,7 +568,7 @@ __global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
   __syncthreads();
   if (p.trace != nullptr) tr.mark(1);
 
-  // 5. combine in slot order
+  // 4. combine in slot order
   if (p.scores != nullptr) {
     if (tid < RB && row0 + tid < H) {
       const uint32_t r = tid;
@@ -602,14 +649,33 @@ hipError_t launch(const char* family, void (*kernel)(KArgs...), dim3 grid, dim3 
   return hipGetLastError();
 }
 
-template <class A, int LPR, int GI, int U>
-hipError_t gateup_go(const GateUpLaunch& p, hipStream_t stream) {
-  constexpr int RPB = (64 / LPR) * U * kGuWaves;
+// Rows of a power of two of groups and a quarter of it over (hidden 2560: 80 =
+// 64 + 16; inter 640: 20 = 16 + 4): a lane takes one group of each whole row,
+// and the quarters over of four rows make one more load of the whole lane
+// group.  With lanes for the next power of two, 38 % of them had no group:
+// hidden 2560 / inter 640, one / five / eight tokens 24.6 / 73.0 / 107.5 us per
+// layer, 21.7 / 63.3 / 85.6 folded (20.7 / 57.1 / 76.9 with 32-bit offsets and
+// the shorter unpacking).
+constexpr int kFold = 4;
+bool quarter_over(uint32_t groups) {
+  const uint32_t whole = next_pow2(groups) / 2;
+  return whole >= 8 && whole <= 64 && groups * kFold == whole * (kFold + 1);
+}
+
+template <class A, int LPR, int GI, int U, int FOLD, int WAVES>
+hipError_t gateup_launch(const GateUpLaunch& p, hipStream_t stream) {
+  constexpr int RPB = (64 / LPR) * U * WAVES;
   const uint32_t pairs = p.tokens * p.slots + (p.has_shared ? p.tokens : 0);
   dim3 grid((p.inter + RPB - 1) / RPB, pairs);
   GateUpLaunch q = p;
   q.trace = trace_reserve(grid.x * grid.y);
-  return launch("gateup", k_gateup<A, LPR, GI, U>, grid, dim3(kGuBlock), stream, q);
+  return launch("gateup", k_gateup<A, LPR, GI, U, FOLD, WAVES>, grid, dim3(WAVES * 64), stream, q);
+}
+
+template <class A, int LPR, int GI, int U, int FOLD = 0>
+hipError_t gateup_go(const GateUpLaunch& p, hipStream_t stream) {
+  if (p.tokens > 1) return gateup_launch<A, LPR, GI, U, FOLD, kGuWavesMulti>(p, stream);
+  return gateup_launch<A, LPR, GI, U, FOLD, kGuWaves>(p, stream);
 }
 
 template <class A>
@@ -617,6 +683,14 @@ hipError_t gateup_dispatch(const GateUpLaunch& p, hipStream_t stream) {
   const uint32_t G = p.hidden / kGroup;
   const uint32_t lpr = G >= 64 ? 64 : next_pow2(G);
   const uint32_t gi = (G + 63) / 64;
+  if (quarter_over(G)) {
+    switch (next_pow2(G) / 2) {
+      case 8: return gateup_go<A, 8, 1, kFold, kFold>(p, stream);
+      case 16: return gateup_go<A, 16, 1, kFold, kFold>(p, stream);
+      case 32: return gateup_go<A, 32, 1, kFold, kFold>(p, stream);
+      default: return gateup_go<A, 64, 1, kFold, kFold>(p, stream);
+    }
+  }
   switch (lpr) {
     case 1: return gateup_go<A, 1, 1, 1>(p, stream);
     case 2: return gateup_go<A, 2, 1, 1>(p, stream);
@@ -631,18 +705,25 @@ hipError_t gateup_dispatch(const GateUpLaunch& p, hipStream_t stream) {
   return gateup_go<A, 64, 4, 1>(p, stream);
 }
 
-template <class A, int LPR>
+template <class A, int LPR, int FOLD = 0, int QUADS = kDownQuads>
 hipError_t down_go(const DownLaunch& p, hipStream_t stream) {
-  constexpr int RB = (64 / LPR) * kDownQuads;
+  constexpr int RB = (64 / LPR) * QUADS;
   dim3 grid((p.hidden + RB - 1) / RB, p.tokens);
   DownLaunch q = p;
   q.trace = trace_reserve(grid.x * grid.y);
-  if (p.inject.out != nullptr) return launch("down", k_down<A, LPR, true>, grid, dim3(kDownBlock), stream, q);
-  return launch("down", k_down<A, LPR, false>, grid, dim3(kDownBlock), stream, q);
+  if (p.inject.out != nullptr) return launch("down", k_down<A, LPR, true, FOLD, QUADS>, grid, dim3(kDownBlock), stream, q);
+  return launch("down", k_down<A, LPR, false, FOLD, QUADS>, grid, dim3(kDownBlock), stream, q);
 }
 
 template <class A>
 hipError_t down_dispatch(const DownLaunch& p, hipStream_t stream) {
+  if (quarter_over(p.inter / kGroup)) {  // at most 64 groups: whole rows of up to 32
+    switch (next_pow2(p.inter / kGroup) / 2) {
+      case 8: return down_go<A, 8, kFold, kFold>(p, stream);
+      case 16: return down_go<A, 16, kFold, kFold>(p, stream);
+      default: return down_go<A, 32, kFold, kFold>(p, stream);
+    }
+  }
   switch (next_pow2(p.inter / kGroup)) {
     case 1: return down_go<A, 1>(p, stream);
     case 2: return down_go<A, 2>(p, stream);

@@ -242,21 +242,28 @@ __device__ __forceinline__ void pair_activations(const uint32_t raw[16], uint32_
   }
 }
 
+// Sum of a group's 32 activations, v_dot2 with pairs of ones: one instruction
+// per pair where unpacking and adding takes four.
 __device__ __forceinline__ float bf16_pair_sum(const uint32_t raw[16]) {
-  float s = 0.0f;
+  const bf16x2 ones = __builtin_bit_cast(bf16x2, 0x3f803f80u);
+  float s[2] = {0.0f, 0.0f};
 #pragma unroll
-  for (int m = 0; m < 16; ++m) s += bf16_to_f32(raw[m] & 0xffffu) + bf16_to_f32(raw[m] >> 16);
-  return s;
+  for (int m = 0; m < 16; ++m)
+    s[m & 1] = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, raw[m]), ones, s[m & 1], false);
+  return s[0] + s[1];
 }
 
 __device__ __forceinline__ float q4_dot_bf16(const uint4 w, const uint32_t xp[16]) {
   const uint32_t words[4] = {w.x, w.y, w.z, w.w};
+  // in a VGPR, so that mask and magic are one v_and_or_b32 (two literals need two instructions)
+  uint32_t magic;
+  asm("v_mov_b32 %0, 0x43004300" : "=v"(magic));
   float acc = 0.0f;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
 #pragma unroll
     for (int n = 0; n < 4; ++n) {
-      const uint32_t q = ((words[i] >> (4 * n)) & 0x000f000fu) | 0x43004300u;
+      const uint32_t q = ((words[i] >> (4 * n)) & 0x000f000fu) | magic;
       acc = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, q),
                                            __builtin_bit_cast(bf16x2, xp[4 * i + n]), acc, false);
     }
