@@ -405,3 +405,22 @@ def test_down_gemm_half_chunk_tail(device, tokens, inter):
     torch.cuda.synchronize()
     _, _, _, d_out, _ = mo.execute(x_np, inds, np_packs, "bf16", qmm=True)
     _close_qmm(host(out), d_out, f"inter {inter}, {tokens} rows")
+
+
+@pytest.mark.parametrize("inter", [256, 640])
+@pytest.mark.parametrize("tokens", [65, 128, 129])
+def test_down_row_tiles_of_larger_calls(device, tokens, inter):
+    """Calls above 64 rows whose experts average up to 16 rows run 16-row down tiles at these widths (24 experts
+    top-3: up to 128 rows; 129 take the chunked GEMM).  One expert gets two thirds of the rows, so it has several
+    tiles and a ragged last one; the last expert's weights end the bank."""
+    hidden, experts, k = 384, 24, 3
+    np_packs = packs(73, hidden, inter, experts)
+    rng = np.random.default_rng(74 + inter + tokens)
+    inds = np.stack([rng.choice(experts, k, replace=False) for _ in range(tokens)]).astype(np.int32)
+    inds[:2 * tokens // 3, 0] = experts - 1
+    x_np = mo.bf16r(rng.normal(size=(tokens, hidden)).astype(np.float32))
+    switch = _switch(np_packs, hidden, inter, experts, device)
+    out = grouped_experts(switch, bf16_device(x_np, device), torch.tensor(inds, device=device))
+    torch.cuda.synchronize()
+    _, _, _, d_out, _ = mo.execute(x_np, inds, np_packs, "bf16", qmm=True)
+    _close_qmm(host(out), d_out, f"inter {inter}, {tokens} rows")

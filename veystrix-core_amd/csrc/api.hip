@@ -526,7 +526,7 @@ struct GroupedWs {
   uint64_t logits, sig, inds, scores, row_off, tiles, tile_count, tiles_dn, tile_count_dn, sort_counts,
       sort_cursors, row_token, pair_row, act, rows, total;
   uint32_t rows_total, groups, max_tiles, max_tiles_dn, tile_rows, tile_rows_dn;
-  bool small;  // 16-row tile kernels (k_rows)
+  bool small, small_dn;  // 16-row tile kernels (k_rows) for gate/up and down
 };
 
 // Calls of up to this many tokens run the 16-row tile kernels, whose blocks
@@ -542,8 +542,22 @@ constexpr uint32_t kRowsMaxTokens = 64;
 #ifndef VM_ROUTER_RING
 #define VM_ROUTER_RING 1
 #endif
-static bool small_grouped(uint32_t T, uint32_t H, uint32_t I) {
-  return VM_ROWS_PATH && T <= kRowsMaxTokens && vm::rows_supported(H) && vm::rows_supported(I);
+static bool small_gateup(uint32_t T, uint32_t H) {
+  return VM_ROWS_PATH && T <= kRowsMaxTokens && vm::rows_gateup_supported(H);
+}
+
+// The down GEMM also in larger calls whose experts average no more rows than
+// one tile, where its chunked GEMM is at its worst: intermediate sizes of one
+// K chunk (nothing to overlap its loads with) or with half a chunk over (three
+// chunks loaded for two and a half).  Hidden 2560 / inter 640, 512 experts
+// top-10, 96 / 333 / 700 rows: 363 / 450 / 487 us per call chunked, 349 / 422 /
+// 466 with 16-row tiles; 1024 / 256, 64 experts top-4, 96 / 256 rows: 37.1 /
+// 40.1 and 35.3 / 38.2.  At inter 512 (two whole chunks) the chunked GEMM
+// keeps these calls: 96 / 333 rows 213 / 265 us against 225 / 274.
+static bool small_down(uint32_t T, uint32_t K, uint32_t I, uint32_t E) {
+  if (!VM_ROWS_PATH || !vm::rows_down_supported(I)) return false;
+  return T <= kRowsMaxTokens ||
+         (uint64_t(T) * K <= uint64_t(E) * vm::kRowsTile && (I == 8 * 32 || vm::down_half_tail(I)));
 }
 
 // Rows per gate/up tile of a chunked-GEMM call: tall tiles when the routed
@@ -563,13 +577,14 @@ static uint32_t down_tile_rows(uint32_t T, uint32_t K, uint32_t I, uint32_t E) {
   return tall ? vm::kGroupedRowsTall : vm::kGroupedRowsDown;
 }
 
-static GroupedWs grouped_ws(uint32_t T, uint32_t K, uint32_t H, uint32_t I, uint32_t E, bool shared) {
+static GroupedWs grouped_ws_of(uint32_t T, uint32_t K, uint32_t H, uint32_t I, uint32_t E, bool shared, bool small_dn) {
   GroupedWs w{};
   w.rows_total = T * K + (shared ? T : 0);
   w.groups = E + (shared ? 1 : 0);
-  w.small = small_grouped(T, H, I);
+  w.small = small_gateup(T, H);
+  w.small_dn = small_dn;
   w.tile_rows = w.small ? vm::kRowsTile : gateup_tile_rows(T, K, H, E);
-  w.tile_rows_dn = w.small ? vm::kRowsTile : down_tile_rows(T, K, I, E);
+  w.tile_rows_dn = w.small_dn ? vm::kRowsTile : down_tile_rows(T, K, I, E);
   w.max_tiles = vm::grouped_max_tiles(w.rows_total, w.groups, w.tile_rows);
   w.max_tiles_dn = vm::grouped_max_tiles(w.rows_total, w.groups, w.tile_rows_dn);
   uint64_t o = kAlign;
@@ -597,6 +612,16 @@ static GroupedWs grouped_ws(uint32_t T, uint32_t K, uint32_t H, uint32_t I, uint
   w.rows = take(uint64_t(w.rows_total) * H * 2);
   w.total = o;
   return w;
+}
+
+// The tile list of 16-row down tiles is a little longer: a call that fits the
+// static scratch without them keeps fitting it.
+static GroupedWs grouped_ws(uint32_t T, uint32_t K, uint32_t H, uint32_t I, uint32_t E, bool shared) {
+  const bool small_dn = small_down(T, K, I, E);
+  const GroupedWs w = grouped_ws_of(T, K, H, I, E, shared, small_dn);
+  if (!small_dn || w.total <= VM_STATIC_SCRATCH_BYTES) return w;
+  const GroupedWs chunked = grouped_ws_of(T, K, H, I, E, shared, false);
+  return chunked.total <= VM_STATIC_SCRATCH_BYTES ? chunked : w;
 }
 
 static bool use_grouped(uint32_t T, uint32_t dtype) { return T > VM_LAYER_MAX_TOKENS && dtype == VM_BF16; }
@@ -1176,10 +1201,10 @@ static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char
   q.a_stride = g.I;
   q.a_rows = g.T * g.K + (g.shared ? g.T : 0);
   q.weights_once = uint64_t(g.T) * g.K <= uint64_t(g.E) * vm::kGroupedRowsDown;
-  q.tile_rows = w.small || w.tile_rows_dn == vm::kGroupedRowsDown ? 0u : w.tile_rows_dn;
+  q.tile_rows = w.small_dn || w.tile_rows_dn == vm::kGroupedRowsDown ? 0u : w.tile_rows_dn;
   q.tiles = s.tiles_dn;
   q.tile_count = s.tile_count_dn;
-  e = w.small ? vm::launch_rows(vm::kEpiRows, q, w.max_tiles_dn, stream)
+  e = w.small_dn ? vm::launch_rows(vm::kEpiRows, q, w.max_tiles_dn, stream)
               : vm::launch_grouped(vm::kEpiRows, q, w.max_tiles_dn, stream);
   if (e != hipSuccess) return hip_fail(e, "grouped down launch");
 
