@@ -419,10 +419,21 @@ constexpr int kDownQuads = VM_DOWN_QUADS;                 // row groups of 64/LP
 // a separate instance, so the plain kernel carries none of its loads.
 // FOLD: rows of LPR (1 + 1 / FOLD) groups (quarter_over).
 template <class A, int LPR, bool INJ, int FOLD, int QUADS>
-__global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
+__global__ __launch_bounds__(kDownBlock, FOLD && !INJ && A::kBytes == 2 ? 6 : 3) void k_down(DownLaunch p) {
   constexpr int RPI = 64 / LPR;
   constexpr int RB = RPI * QUADS;
-  constexpr int NX = FOLD ? 2 : 1;                          // activation groups per lane and slot
+  // FOLD: a lane needs two activation groups of its slot.  Kept in registers
+  // through the wait for the weights they cost the block its second place on
+  // the CU (12 waves at 86 VGPRs), so the wave keeps its slot's activations in
+  // LDS (16 bytes of padding per group: the lanes' reads are conflict-free) and
+  // takes one group at a time: 80 VGPRs; hidden 2560 / inter 640, one / five /
+  // eight tokens 20.9 / 57.5 / 76.9 -> 20.3 / 52.1 / 70.0 us per layer.
+  constexpr int kUPG = kGroup * A::kBytes / 16;             // 16-byte units per group
+  constexpr int kActG = FOLD ? LPR + LPR / (FOLD + !FOLD) : 1;  // groups of a row
+  constexpr int kActU = (kActG * kUPG + 63) / 64;           // units per lane
+  constexpr int kGroupBytes = kUPG * 16 + 16;
+  __shared__ __align__(16) uint8_t s_act[FOLD ? kDownWaves : 1][kActG * kGroupBytes];
+  static_assert(FOLD == 0 || kDownSlotsPerWave == 1, "one slot's activations per wave");
   constexpr int NF = FOLD ? (QUADS + FOLD - 1) / FOLD : 0;  // folded loads per lane and slot
   constexpr int REM = FOLD ? LPR / FOLD : 1;                // groups over of a row
   __shared__ float s_part[kDownMaxSlots * RB];
@@ -456,15 +467,19 @@ __global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
   //    wave's activation groups (slot wave + 4 i, group lr)
   const uint32_t route = ldg_u32(p.routes + static_cast<size_t>(t) * K + min(lane, K - 1));
   asm volatile("" ::: "memory");
-  GroupAct<A> xa[kDownSlotsPerWave][NX];
+  GroupAct<A> xa[kDownSlotsPerWave];
+  uint4 act[kActU];
+  if constexpr (FOLD > 0) {
+    const uint8_t* src = static_cast<const uint8_t*>(p.act) +
+                         (static_cast<size_t>(t) * S + min(wave, S - 1)) * I * A::kBytes;
 #pragma unroll
-  for (int i = 0; i < kDownSlotsPerWave; ++i) {
-    const uint32_t slot = wave + kDownWaves * i;
+    for (int i = 0; i < kActU; ++i) act[i] = ldg16(src + min(lane + 64u * i, kActG * kUPG - 1u) * 16u);
+  } else {
 #pragma unroll
-    for (int x = 0; x < NX; ++x) {
-      const uint32_t g = x ? LPR + lr % REM : lr;
-      const bool live = slot < S && g < G;
-      xa[i][x].fetch(live ? p.act : g_zero_page, live ? (static_cast<size_t>(t) * S + slot) * I + g * kGroup : 0);
+    for (int i = 0; i < kDownSlotsPerWave; ++i) {
+      const uint32_t slot = wave + kDownWaves * i;
+      const bool live = slot < S && lr < G;
+      xa[i].fetch(live ? p.act : g_zero_page, live ? (static_cast<size_t>(t) * S + slot) * I + lr * kGroup : 0);
     }
   }
 
@@ -541,6 +556,17 @@ __global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
     }
   }
   if (p.trace != nullptr) tr.mark(6);
+  if constexpr (FOLD > 0) {
+#pragma unroll
+    for (int i = 0; i < kActU; ++i) {
+      const uint32_t u = min(lane + 64u * i, kActG * kUPG - 1u);  // lanes past the end repeat the last unit
+      *reinterpret_cast<uint4*>(&s_act[wave][(u / kUPG) * kGroupBytes + (u % kUPG) * 16]) = act[i];
+    }
+    // read by other lanes of this wave only: LDS works in order within a wave
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  }
   if (p.trace != nullptr) tr.mark(7);
 
   // 3. dot products and row sums into LDS
@@ -548,16 +574,21 @@ __global__ __launch_bounds__(kDownBlock) void k_down(DownLaunch p) {
   for (int i = 0; i < kDownSlotsPerWave; ++i) {
     const uint32_t slot = wave + kDownWaves * i;
     if (slot >= S) break;  // wave-uniform
-#pragma unroll
-    for (int x = 0; x < NX; ++x) xa[i][x].prepare();
     float over[NF + !NF];
+    if constexpr (FOLD > 0) {
+      GroupAct<A> xf;
+      xf.fetch(&s_act[wave][(LPR + lr % REM) * kGroupBytes], 0);
+      xf.prepare();
 #pragma unroll
-    for (int f = 0; f < NF; ++f)
-      over[f] = xa[i][NX - 1].apply(w[i][QUADS + f], bf16_to_f32(sc[i][QUADS + f]), bf16_to_f32(bi[i][QUADS + f]));
+      for (int f = 0; f < NF; ++f)
+        over[f] = xf.apply(w[i][QUADS + f], bf16_to_f32(sc[i][QUADS + f]), bf16_to_f32(bi[i][QUADS + f]));
+      xa[i].fetch(&s_act[wave][lr * kGroupBytes], 0);
+    }
+    xa[i].prepare();
 #pragma unroll
     for (int q = 0; q < QUADS; ++q) {
       const uint32_t has = FOLD || lr < G ? ~0u : 0u;
-      float v = xa[i][0].apply(w[i][q], bf16_to_f32(sc[i][q] & has), bf16_to_f32(bi[i][q] & has));
+      float v = xa[i].apply(w[i][q], bf16_to_f32(sc[i][q] & has), bf16_to_f32(bi[i][q] & has));
       if constexpr (FOLD > 0) v += lr / REM == static_cast<uint32_t>(q % FOLD) ? over[q / FOLD] : 0.0f;
       v = group_sum<LPR>(v);
       if (lr == LPR - 1) s_part[slot * RB + q * RPI + rw] = v;
@@ -655,7 +686,7 @@ hipError_t launch(const char* family, void (*kernel)(KArgs...), dim3 grid, dim3 
 // group.  With lanes for the next power of two, 38 % of them had no group:
 // hidden 2560 / inter 640, one / five / eight tokens 24.6 / 73.0 / 107.5 us per
 // layer, 21.7 / 63.3 / 85.6 folded (20.7 / 57.1 / 76.9 with 32-bit offsets and
-// the shorter unpacking).
+// the shorter unpacking, 20.3 / 52.1 / 70.0 with down's activations in LDS).
 constexpr int kFold = 4;
 bool quarter_over(uint32_t groups) {
   const uint32_t whole = next_pow2(groups) / 2;
