@@ -731,6 +731,10 @@ hipError_t gateup_dispatch(const GateUpLaunch& p, hipStream_t stream) {
     case 32: return gateup_go<A, 32, 1, 2>(p, stream);
     default: break;
   }
+  // three tokens and more fill the chip with four rows per wave too, and half as
+  // many blocks repeat the selection (hidden 2048, 3 / 5 / 8 tokens 26.9 / 38.6 /
+  // 52.8 -> 25.0 / 36.9 / 50.5 us per layer, two tokens 20.3 -> 20.4)
+  if (gi <= 1 && p.tokens > 2) return gateup_launch<A, 64, 1, 2 * kGateupRowsPerLane, 0, kGuWavesMulti>(p, stream);
   if (gi <= 1) return gateup_go<A, 64, 1, kGateupRowsPerLane>(p, stream);
   if (gi <= 2) return gateup_go<A, 64, 2, 2>(p, stream);
   return gateup_go<A, 64, 4, 1>(p, stream);
