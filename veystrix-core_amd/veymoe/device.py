@@ -19,7 +19,7 @@ def require_device(name: str, tensor, dtypes=None):
     """Check that ``tensor`` is a contiguous tensor on the GPU (optionally of a dtype)."""
     if not isinstance(tensor, torch.Tensor):
         raise TypeError(f"{name} must be a torch tensor on the GPU, got {type(tensor).__name__}")
-    if tensor.device.type != "cuda":
+    if not tensor.is_cuda:
         raise TypeError(f"{name} must live on the GPU (got {tensor.device})")
     if not tensor.is_contiguous():
         raise ValueError(f"{name} must be contiguous")
@@ -50,7 +50,10 @@ def word_tensor(name: str, tensor):
 
 
 def stream_handle(stream=None) -> ctypes.c_void_p:
-    stream = torch.cuda.current_stream() if stream is None else stream
+    if stream is None:
+        # the raw handle of torch.cuda.current_stream(), without the Stream
+        # object (2.9 us of a call's 20 us on the host)
+        return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
     return ctypes.c_void_p(stream.cuda_stream)
 
 

@@ -387,8 +387,9 @@ class MoELayer:
     @staticmethod
     def _set_inject(args, flat: torch.Tensor, inject) -> None:
         if inject is None:
-            args.inject_hidden = args.inject_weights = args.inject_out = None
-            args.hc_count = 0
+            if args.inject_out is not None:  # the arguments of an earlier call with an injection
+                args.inject_hidden = args.inject_weights = args.inject_out = None
+                args.hc_count = 0
             return
         streams, weights, target = inject
         rows = flat.shape[0]
@@ -422,6 +423,8 @@ class MoELayer:
     prefill = forward
 
     def __call__(self, x: torch.Tensor) -> torch.Tensor:
+        if x.dim() == 2 and x.is_contiguous():
+            return self.forward(x)
         hidden = x.shape[-1]
         flat = x.reshape(-1, hidden).contiguous()
         return self.forward(flat).reshape(x.shape)
