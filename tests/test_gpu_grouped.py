@@ -408,19 +408,24 @@ def test_down_gemm_half_chunk_tail(device, tokens, inter):
 
 
 @pytest.mark.parametrize("inter", [256, 640])
-@pytest.mark.parametrize("tokens", [65, 128, 129])
-def test_down_row_tiles_of_larger_calls(device, tokens, inter):
-    """Calls above 64 rows whose experts average up to 16 rows run 16-row down tiles at these widths (24 experts
-    top-3: up to 128 rows; 129 take the chunked GEMM).  One expert gets two thirds of the rows, so it has several
-    tiles and a ragged last one; the last expert's weights end the bank."""
-    hidden, experts, k = 384, 24, 3
+@pytest.mark.parametrize("hidden", [96, 1088])
+def test_down_gemm_of_whole_rows_gives_the_chunked_bits(device, hidden, inter):
+    """At these widths calls of up to 48 rows per expert keep a tile's whole rows in LDS (k_down_rows), calls above
+    take the chunked GEMM's 96-row tiles: the same tokens give the same bits in both, and match the oracle.  Two
+    thirds of the rows go to the last expert (several tiles, a ragged last one, the bank's end); output widths that
+    end inside a block and inside its second pass."""
+    experts, k = 24, 3
     np_packs = packs(73, hidden, inter, experts)
-    rng = np.random.default_rng(74 + inter + tokens)
-    inds = np.stack([rng.choice(experts, k, replace=False) for _ in range(tokens)]).astype(np.int32)
+    rng = np.random.default_rng(74 + inter + hidden)
+    tokens, more = 150, 500
+    inds = np.stack([rng.choice(experts - 1, k, replace=False) for _ in range(more)]).astype(np.int32)
     inds[:2 * tokens // 3, 0] = experts - 1
-    x_np = mo.bf16r(rng.normal(size=(tokens, hidden)).astype(np.float32))
+    x_np = mo.bf16r(rng.normal(size=(more, hidden)).astype(np.float32))
     switch = _switch(np_packs, hidden, inter, experts, device)
-    out = grouped_experts(switch, bf16_device(x_np, device), torch.tensor(inds, device=device))
+    x, i = bf16_device(x_np, device), torch.tensor(inds, device=device)
+    out = grouped_experts(switch, x[:tokens].contiguous(), i[:tokens].contiguous())
+    tall = grouped_experts(switch, x, i)
     torch.cuda.synchronize()
-    _, _, _, d_out, _ = mo.execute(x_np, inds, np_packs, "bf16", qmm=True)
-    _close_qmm(host(out), d_out, f"inter {inter}, {tokens} rows")
+    _, _, _, d_out, _ = mo.execute(x_np[:tokens], inds[:tokens], np_packs, "bf16", qmm=True)
+    _close_qmm(host(out), d_out, f"hidden {hidden}, inter {inter}")
+    assert torch.equal(out.view(torch.int16), tall[:tokens].view(torch.int16))

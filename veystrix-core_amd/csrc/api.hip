@@ -546,18 +546,8 @@ static bool small_gateup(uint32_t T, uint32_t H) {
   return VM_ROWS_PATH && T <= kRowsMaxTokens && vm::rows_gateup_supported(H);
 }
 
-// The down GEMM also in larger calls whose experts average no more rows than
-// one tile, where its chunked GEMM is at its worst: intermediate sizes of one
-// K chunk (nothing to overlap its loads with) or with half a chunk over (three
-// chunks loaded for two and a half).  Hidden 2560 / inter 640, 512 experts
-// top-10, 96 / 333 / 700 rows: 363 / 450 / 487 us per call chunked, 349 / 422 /
-// 466 with 16-row tiles; 1024 / 256, 64 experts top-4, 96 / 256 rows: 37.1 /
-// 40.1 and 35.3 / 38.2.  At inter 512 (two whole chunks) the chunked GEMM
-// keeps these calls: 96 / 333 rows 213 / 265 us against 225 / 274.
-static bool small_down(uint32_t T, uint32_t K, uint32_t I, uint32_t E) {
-  if (!VM_ROWS_PATH || !vm::rows_down_supported(I)) return false;
-  return T <= kRowsMaxTokens ||
-         (uint64_t(T) * K <= uint64_t(E) * vm::kRowsTile && (I == 8 * 32 || vm::down_half_tail(I)));
+static bool small_down(uint32_t T, uint32_t I) {
+  return VM_ROWS_PATH && T <= kRowsMaxTokens && vm::rows_down_supported(I);
 }
 
 // Rows per gate/up tile of a chunked-GEMM call: tall tiles when the routed
@@ -571,7 +561,9 @@ static uint32_t gateup_tile_rows(uint32_t T, uint32_t K, uint32_t H, uint32_t E)
 }
 
 // Rows per down tile: the same rule over the intermediate size and the down
-// GEMM's usual height (3072 rows 514-519 -> 502-508 us per call).
+// GEMM's usual height (3072 rows 514-519 -> 502-508 us per call; at inter 640,
+// where tiles of the usual height run k_down_rows, 3000 / 4096 rows take 713 /
+// 818 us with tall tiles and 731 / 840 without).
 static uint32_t down_tile_rows(uint32_t T, uint32_t K, uint32_t I, uint32_t E) {
   const bool tall = uint64_t(T) * K > uint64_t(E) * vm::kGroupedRowsDown && vm::down_tall_supported(I);
   return tall ? vm::kGroupedRowsTall : vm::kGroupedRowsDown;
@@ -617,7 +609,7 @@ static GroupedWs grouped_ws_of(uint32_t T, uint32_t K, uint32_t H, uint32_t I, u
 // The tile list of 16-row down tiles is a little longer: a call that fits the
 // static scratch without them keeps fitting it.
 static GroupedWs grouped_ws(uint32_t T, uint32_t K, uint32_t H, uint32_t I, uint32_t E, bool shared) {
-  const bool small_dn = small_down(T, K, I, E);
+  const bool small_dn = small_down(T, I);
   const GroupedWs w = grouped_ws_of(T, K, H, I, E, shared, small_dn);
   if (!small_dn || w.total <= VM_STATIC_SCRATCH_BYTES) return w;
   const GroupedWs chunked = grouped_ws_of(T, K, H, I, E, shared, false);
@@ -1205,7 +1197,9 @@ static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char
   q.tiles = s.tiles_dn;
   q.tile_count = s.tile_count_dn;
   e = w.small_dn ? vm::launch_rows(vm::kEpiRows, q, w.max_tiles_dn, stream)
-              : vm::launch_grouped(vm::kEpiRows, q, w.max_tiles_dn, stream);
+      : w.tile_rows_dn == vm::kGroupedRowsDown && vm::down_rows_supported(g.I)
+          ? vm::launch_down_rows(q, w.max_tiles_dn, stream)
+          : vm::launch_grouped(vm::kEpiRows, q, w.max_tiles_dn, stream);
   if (e != hipSuccess) return hip_fail(e, "grouped down launch");
 
   vm::CombineLaunch c{};

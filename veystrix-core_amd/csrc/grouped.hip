@@ -1128,6 +1128,173 @@ __global__ __launch_bounds__(WAVES * 64) void k_rows(GroupedLaunch p) {
   }
 }
 
+// ------------------------------------------------- down GEMM, whole rows ---
+
+// The down GEMM of tiles of up to 48 rows at intermediate sizes of up to 640:
+// the block stages its tile's A rows over the whole K in LDS once, as k_rows
+// does, and every wave streams the weights of SPB column blocks of 16 straight
+// into its MFMA lanes, the next block's loads in flight while one is
+// multiplied, with no barrier after the staging.  The chunked GEMM passes the
+// weights through LDS, two barriers per chunk and a load latency that two or
+// three chunks of K hardly cover; here a dequantised operand feeds as many
+// MFMAs and nothing but the wave's own loads is waited for.  Bound by HBM:
+// hidden 2560 / inter 640, 512 experts top-10, 333 / 1000 / 1999 / 2400 rows:
+// 450 / 504 / 599 / 669 us per call chunked, 402 / 456 / 549 / 607 so (16-row
+// tiles at 333 rows: 416); hidden 1024 / inter 256, 64 experts top-4, 333 rows:
+// 41.8 and 38.8.  At inter 512, two whole chunks, it is the slower one (1999
+// rows 352 and 363 us).
+//
+// K order is the chunked GEMM's: MFMA step (g, i) feeds k block kb from group
+// 4 g + kb, packed word i, so both give the same bits and a row's result does
+// not depend on which of the two its call takes.  The 16-byte unit u of A row
+// r sits at unit u ^ (r mod 16) of its 16-unit block.  A column's scales lie
+// together: its four lanes load 16 bytes of them each (the last ones
+// overlapping) and pass them through a strip of LDS of the wave's own, where
+// each lane finds its groups (a 2-byte load per group and lane from 16 rows of
+// scales costs more than the weights).
+template <int QG>
+struct DownB {
+  static constexpr uint32_t kMeta = 4 * QG * 2;                // bytes of a column's scales
+  static constexpr uint32_t kStrip = (kMeta + 15) / 16 * 16;   // the same in LDS
+  uint4 w[QG], s, b;
+  __device__ __forceinline__ void load(const ProjPtrs& p, uint32_t col, uint32_t q) {
+    const uint32_t at = col * kMeta + min(q * 16u, kMeta - 16u);
+    s = ldg16(reinterpret_cast<const uint8_t*>(p.s) + at);
+    b = ldg16(reinterpret_cast<const uint8_t*>(p.b) + at);
+#pragma unroll
+    for (int g = 0; g < QG; ++g)
+      w[g] = ldg16(reinterpret_cast<const uint8_t*>(p.w) + (col * (4u * QG) + q) * 16u + g * 64u);
+  }
+  __device__ __forceinline__ static void put(uint8_t* strip, const uint4& v, uint32_t q) {
+    uint2* dst = reinterpret_cast<uint2*>(strip + min(q * 16u, kMeta - 16u));
+    dst[0] = make_uint2(v.x, v.y);
+    dst[1] = make_uint2(v.z, v.w);
+  }
+};
+
+template <int QG, int WAVES, int SPB, int MBU>
+__device__ __forceinline__ void down_rows_tile(const GroupedLaunch& p, const ProjPtrs& w, uint32_t row0, uint32_t rows,
+                                               uint32_t slice0, uint8_t* s_a) {
+  constexpr int kThreads = WAVES * 64;
+  constexpr int kUnits = QG * 16;  // 16-byte A units per row
+  constexpr int kRowBytes = kUnits * 16;
+  using B = DownB<QG>;
+  constexpr int kIt = (MBU * 16 * kUnits + kThreads - 1) / kThreads;
+  const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const uint32_t N = p.n_dim;
+  const uint32_t bn = lane & 15u, q = lane >> 4;
+  // A rows of the tile: contiguous; rows past the tile repeat its last one
+  // (an MFMA output row depends on its own A row only, and those are not stored)
+  uint4 av[kIt];
+  const uint8_t* a0 = reinterpret_cast<const uint8_t*>(p.a) + static_cast<size_t>(row0) * kRowBytes;
+  const auto unit = [&](int j) { return min(j * kThreads + tid, static_cast<uint32_t>(MBU * 16 * kUnits - 1)); };
+#pragma unroll
+  for (int j = 0; j < kIt; ++j) {
+    const uint32_t it = unit(j), r = min(it / kUnits, rows - 1), u = it % kUnits;
+    av[j] = ldg16(a0 + r * static_cast<uint32_t>(kRowBytes) + u * 16u);
+  }
+  // columns past N read the last row and are not stored
+  const auto column = [&](int s) { return ((slice0 + s) * WAVES + wave) * 16u + bn; };
+  B b[2];
+  b[0].load(w, min(column(0), N - 1), q);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < kIt; ++j) {
+    const uint32_t it = unit(j), r = it / kUnits, u = it % kUnits;
+    *reinterpret_cast<uint4*>(s_a + r * kRowBytes + (u ^ (r & 15u)) * 16u) = av[j];
+  }
+  __syncthreads();
+  const uint32_t magic = f16_magic();
+  const uint8_t* a_lane = s_a + bn * kRowBytes;
+  // the wave's strips of scales and biases, column bn's
+  uint8_t* strip = s_a + kGroupedRowsDown * kRowBytes + (wave * 32u + bn) * B::kStrip;
+#pragma unroll
+  for (int s = 0; s < SPB; ++s) {
+    if (s + 1 < SPB) {
+      b[(s + 1) & 1].load(w, min(column(s + 1), N - 1), q);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const B& bs = b[s & 1];
+    B::put(strip, bs.s, q);
+    B::put(strip + 16u * B::kStrip, bs.b, q);
+    // read by other lanes of this wave only: LDS works in order within a wave
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    f32x4_t acc[MBU];
+#pragma unroll
+    for (int mb = 0; mb < MBU; ++mb) acc[mb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int g = 0; g < QG; ++g) {
+      const uint32_t at = (4u * g + q) * 2u;
+      const Dequant dq(bf16_to_f32(*reinterpret_cast<const uint16_t*>(strip + at)),
+                       bf16_to_f32(*reinterpret_cast<const uint16_t*>(strip + 16u * B::kStrip + at)));
+#pragma unroll
+      for (int st = 0; st < 4; ++st) {
+        const uint32_t phys = 16u * g + ((4u * q + st) ^ bn);
+        uint32_t r4[4];
+        dq.word(st == 0 ? bs.w[g].x : st == 1 ? bs.w[g].y : st == 2 ? bs.w[g].z : bs.w[g].w, magic, r4);
+        const bf16x8_t bop = as_operand(r4);
+#pragma unroll
+        for (int mb = 0; mb < MBU; ++mb) {
+          const bf16x8_t aop =
+              __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(a_lane + mb * 16 * kRowBytes + phys * 16u));
+          acc[mb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aop, bop, acc[mb], 0, 0, 0);
+        }
+      }
+    }
+    const uint32_t col = column(s);
+    if (col < N) {
+#pragma unroll
+      for (int mb = 0; mb < MBU; ++mb) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t r = mb * 16 + 4 * q + i;
+          if (r < rows) ActBF16::store(p.out, (row0 + r) * N + col, round_bf16(acc[mb][i]));
+        }
+      }
+    }
+  }
+}
+
+template <int QG, int WAVES, int SPB>
+__global__ __launch_bounds__(WAVES * 64, 4) void k_down_rows(GroupedLaunch p) {
+  extern __shared__ uint4 s_dyn[];
+  uint8_t* s_a = reinterpret_cast<uint8_t*>(s_dyn);
+  const uint32_t tid = threadIdx.x, N = p.n_dim;
+  // XCD-aware order, as the chunked GEMM's: each XCD takes a contiguous run of
+  // the tiles with all their column slices
+  const uint32_t slices = (N + WAVES * 16 * SPB - 1) / (WAVES * 16 * SPB);
+  const uint32_t lin = blockIdx.x, local = (lin >> 3) / slices, slice0 = (lin >> 3) % slices * SPB;
+  const uint32_t count = *p.tile_count, chunk = (count + 7) / 8;
+  const uint32_t tile = (lin & 7u) * chunk + local;
+  if (local >= chunk || tile >= count) return;
+  const uint2 td = p.tiles[tile];
+  const uint32_t group = td.x;
+  const uint32_t row0 = p.row_off[group] + td.y;
+  const uint32_t rows = min(p.row_off[group + 1] - row0, static_cast<uint32_t>(kGroupedRowsDown));
+  ProjPtrs w = p.shared[0];
+  bool ok = w.w != nullptr;
+  if (group < p.experts) {
+    uint32_t index = 0;
+    const int kind = resolve_word(group, p.slot_table, p.experts, p.pool, &p.stream, p.dense[0].w != nullptr, index);
+    ok = kind != kSrcNone;
+    source_proj(kind, index, p.pool, &p.stream, p.dense[0], p.part[0], N, p.k_dim, w);
+  }
+  if (!ok) {  // an unresolved expert: its rows are zero (status flagged)
+    if (tid == 0 && slice0 == 0) flag(p.status, 1u);
+    constexpr uint32_t cols = WAVES * 16 * SPB;
+    for (uint32_t i = tid; i < rows * cols; i += WAVES * 64) {
+      const uint32_t col = slice0 * WAVES * 16 + i % cols;
+      if (col < N) ActBF16::store(p.out, static_cast<size_t>(row0 + i / cols) * N + col, 0.0f);
+    }
+    return;
+  }
+  if (rows > 32) down_rows_tile<QG, WAVES, SPB, 3>(p, w, row0, rows, slice0, s_a);
+  else if (rows > 16) down_rows_tile<QG, WAVES, SPB, 2>(p, w, row0, rows, slice0, s_a);
+  else down_rows_tile<QG, WAVES, SPB, 1>(p, w, row0, rows, slice0, s_a);
+}
+
 // ------------------------------------------------------------------ sort ---
 
 // Inclusive scan of one value per thread over a block of 1024 threads.
@@ -1637,9 +1804,9 @@ hipError_t launch_grouped(int epi, const GroupedLaunch& p, uint32_t max_tiles, h
 // rows (down at 640: 20.4 against 24.9).
 constexpr uint32_t kRowsMaxK = 4096;
 
-bool down_half_tail(uint32_t k_dim) { return half_tail(k_dim / kGroup); }
-
-bool down_tall_supported(uint32_t k_dim) { return (k_dim / kGroup) % kCG == 0 || down_half_tail(k_dim); }
+bool down_tall_supported(uint32_t k_dim) {
+  return (k_dim / kGroup) % kCG == 0 || half_tail(k_dim / kGroup);
+}
 
 bool rows_gateup_supported(uint32_t k_dim) {
   return k_dim == 256 || k_dim == 512 || k_dim == 1024 || k_dim == 2048 || k_dim == kRowsMaxK;
@@ -1696,6 +1863,41 @@ hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipS
   if (epi == kEpiSwiglu) return rows_go<kEpiSwiglu, VM_ROWS_GU_WAVES, 2>("grouped_gateup", p, max_tiles, stream);
   if (epi == kEpiRows) return rows_go<kEpiRows, VM_ROWS_DN_WAVES, 1>("grouped_down", p, max_tiles, stream);
   return hipErrorInvalidValue;
+}
+
+// SPB: column blocks per wave; fewer at the narrow width, whose calls would
+// not fill the chip.
+template <int QG, int SPB>
+hipError_t down_rows_go(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
+  constexpr int kWaves = 8;
+  auto kernel = &k_down_rows<QG, kWaves, SPB>;
+  constexpr uint32_t lds = kGroupedRowsDown * 4u * QG * kGroup * 2u + kWaves * 32u * DownB<QG>::kStrip;
+  static bool attr = false;  // one attribute call per kernel instance
+  if (!attr) {
+    hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+    if (e != hipSuccess) return e;
+    attr = true;
+  }
+  const uint32_t cols = kWaves * 16 * SPB;
+  const dim3 grid(((p.n_dim + cols - 1) / cols) * ((max_tiles + 7) / 8 * 8));
+  hipEvent_t start = nullptr, stop = nullptr;
+  if (timing_events("grouped_down", &start, &stop))
+    hipExtLaunchKernelGGL(kernel, grid, dim3(kWaves * 64), lds, stream, start, stop, 0, p);
+  else
+    hipLaunchKernelGGL(kernel, grid, dim3(kWaves * 64), lds, stream, p);
+  return hipGetLastError();
+}
+
+bool down_rows_supported(uint32_t k_dim) { return k_dim == 256 || k_dim == 640; }
+
+hipError_t launch_down_rows(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
+  if (p.a_stride != p.k_dim || p.row_token != nullptr) return hipErrorInvalidValue;
+  switch (p.k_dim) {
+    case 256: return down_rows_go<2, 2>(p, max_tiles, stream);
+    case 640: return down_rows_go<5, 4>(p, max_tiles, stream);
+    default: return hipErrorInvalidValue;
+  }
 }
 
 hipError_t launch_sort(const SortLaunch& p, hipStream_t stream) {
