@@ -420,12 +420,35 @@ def test_down_gemm_of_whole_rows_gives_the_chunked_bits(device, hidden, inter):
     tokens, more = 150, 500
     inds = np.stack([rng.choice(experts - 1, k, replace=False) for _ in range(more)]).astype(np.int32)
     inds[:2 * tokens // 3, 0] = experts - 1
+    valid = inds[:tokens].copy()
+    inds[5, 2] = 99                          # names no expert: a row of zeros
     x_np = mo.bf16r(rng.normal(size=(more, hidden)).astype(np.float32))
     switch = _switch(np_packs, hidden, inter, experts, device)
     x, i = bf16_device(x_np, device), torch.tensor(inds, device=device)
     out = grouped_experts(switch, x[:tokens].contiguous(), i[:tokens].contiguous())
     tall = grouped_experts(switch, x, i)
     torch.cuda.synchronize()
-    _, _, _, d_out, _ = mo.execute(x_np[:tokens], inds[:tokens], np_packs, "bf16", qmm=True)
+    _, _, _, d_out, _ = mo.execute(x_np[:tokens], valid, np_packs, "bf16", qmm=True)
+    d_out[5, 2] = 0.0
+    assert float(out[5, 2].abs().max()) == 0.0
     _close_qmm(host(out), d_out, f"hidden {hidden}, inter {inter}")
     assert torch.equal(out.view(torch.int16), tall[:tokens].view(torch.int16))
+
+
+def test_slot_rows_of_a_sort_over_many_blocks(device):
+    """One output row per token and slot, stored by the down GEMM itself: 1400 tokens top-3 over 96 experts (more
+    pairs than one sort block takes) give the bits of two calls of 700."""
+    hidden, inter, experts, tokens, k = 128, 256, 96, 1400, 3
+    np_packs = packs(75, hidden, inter, experts)
+    rng = np.random.default_rng(76)
+    inds = torch.tensor(np.stack([rng.choice(experts, k, replace=False) for _ in range(tokens)]).astype(np.int32))
+    inds[900, 1] = -1
+    inds = inds.to(device)
+    x = bf16_device(mo.bf16r(rng.normal(size=(tokens, hidden)).astype(np.float32)), device)
+    switch = _switch(np_packs, hidden, inter, experts, device)
+    whole = grouped_experts(switch, x, inds)
+    halves = torch.cat([grouped_experts(switch, x[:700].contiguous(), inds[:700].contiguous()),
+                        grouped_experts(switch, x[700:].contiguous(), inds[700:].contiguous())])
+    torch.cuda.synchronize()
+    assert float(whole[900, 1].abs().max()) == 0.0
+    assert torch.equal(whole.view(torch.int16), halves.view(torch.int16))

@@ -1193,6 +1193,12 @@ __device__ __forceinline__ void down_rows_tile(const GroupedLaunch& p, const Pro
     const uint32_t it = unit(j), r = min(it / kUnits, rows - 1), u = it % kUnits;
     av[j] = ldg16(a0 + r * static_cast<uint32_t>(kRowBytes) + u * 16u);
   }
+  // the output row of every row of the tile
+  uint32_t* s_out = reinterpret_cast<uint32_t*>(s_a + kGroupedRowsDown * kRowBytes + WAVES * 32u * B::kStrip);
+  if (tid < MBU * 16) {
+    const uint32_t r = row0 + min(tid, rows - 1);
+    s_out[tid] = p.out_row != nullptr ? p.out_row[r] : r;
+  }
   // columns past N read the last row and are not stored
   const auto column = [&](int s) { return ((slice0 + s) * WAVES + wave) * 16u + bn; };
   B b[2];
@@ -1250,7 +1256,7 @@ __device__ __forceinline__ void down_rows_tile(const GroupedLaunch& p, const Pro
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
           const uint32_t r = mb * 16 + 4 * q + i;
-          if (r < rows) ActBF16::store(p.out, (row0 + r) * N + col, round_bf16(acc[mb][i]));
+          if (r < rows) ActBF16::store(p.out, s_out[r] * N + col, round_bf16(acc[mb][i]));
         }
       }
     }
@@ -1286,7 +1292,8 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_down_rows(GroupedLaunch p) {
     constexpr uint32_t cols = WAVES * 16 * SPB;
     for (uint32_t i = tid; i < rows * cols; i += WAVES * 64) {
       const uint32_t col = slice0 * WAVES * 16 + i % cols;
-      if (col < N) ActBF16::store(p.out, static_cast<size_t>(row0 + i / cols) * N + col, 0.0f);
+      const uint32_t r = row0 + i / cols;
+      if (col < N) ActBF16::store(p.out, static_cast<size_t>(p.out_row != nullptr ? p.out_row[r] : r) * N + col, 0.0f);
     }
     return;
   }
@@ -1296,6 +1303,19 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_down_rows(GroupedLaunch p) {
 }
 
 // ------------------------------------------------------------------ sort ---
+
+// Pair i got sorted row pos, or names no expert.  Where the down GEMM stores
+// straight into the caller's rows [pair, hidden] (slot_out) the list holds the
+// pair of every row, and the row of a pair without an expert is zeroed here.
+__device__ __forceinline__ void sort_pair(const SortLaunch& p, uint32_t i, uint32_t pos, bool live) {
+  if (p.slot_out == nullptr) {
+    p.pair_row[i] = live ? pos : kNoRow;
+  } else if (live) {
+    p.pair_row[pos] = i;
+  } else {
+    for (uint32_t h = 0; h < p.hidden; ++h) p.slot_out[static_cast<size_t>(i) * p.hidden + h] = 0;
+  }
+}
 
 // Inclusive scan of one value per thread over a block of 1024 threads.
 __device__ uint32_t block_scan_1024(uint32_t v, uint32_t* s_wave) {
@@ -1369,9 +1389,9 @@ __global__ __launch_bounds__(1024) void k_sort(SortLaunch p) {
     if (e < p.experts) {
       const uint32_t pos = atomicAdd(&s_count[e], 1u);
       p.row_token[pos] = i / p.slots;
-      p.pair_row[i] = pos;
+      sort_pair(p, i, pos, true);
     } else {
-      p.pair_row[i] = kNoRow;
+      sort_pair(p, i, 0, false);
     }
   }
   for (uint32_t i = g; i < p.shared_rows; i += 1024) p.row_token[s_shared_first + i] = i;
@@ -1454,9 +1474,9 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(SortLaunch p) {
     if (e[j] < p.experts) {
       const uint32_t pos = s_base[e[j]] + local[j];
       p.row_token[pos] = i / p.slots;
-      p.pair_row[i] = pos;
+      sort_pair(p, i, pos, true);
     } else {
-      p.pair_row[i] = kNoRow;
+      sort_pair(p, i, 0, false);
     }
   }
 }
@@ -1871,7 +1891,8 @@ template <int QG, int SPB>
 hipError_t down_rows_go(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
   constexpr int kWaves = 8;
   auto kernel = &k_down_rows<QG, kWaves, SPB>;
-  constexpr uint32_t lds = kGroupedRowsDown * 4u * QG * kGroup * 2u + kWaves * 32u * DownB<QG>::kStrip;
+  constexpr uint32_t lds = kGroupedRowsDown * 4u * QG * kGroup * 2u + kWaves * 32u * DownB<QG>::kStrip +
+                           kGroupedRowsDown * 4u;
   static bool attr = false;  // one attribute call per kernel instance
   if (!attr) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
