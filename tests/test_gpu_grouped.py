@@ -452,3 +452,57 @@ def test_slot_rows_of_a_sort_over_many_blocks(device):
     torch.cuda.synchronize()
     assert float(whole[900, 1].abs().max()) == 0.0
     assert torch.equal(whole.view(torch.int16), halves.view(torch.int16))
+
+
+@pytest.mark.parametrize("inter", [256, 640])
+@pytest.mark.parametrize("hidden,tokens", [(96, 70), (1088, 150), (128, 1400)])
+@pytest.mark.parametrize("share", [0.35, 1.0], ids=["third", "all"])
+def test_slot_rows_of_ids_without_an_expert(device, monkeypatch, inter, hidden, tokens, share):
+    """Slot rows of pairs padded with ids that name no expert (-1 and one past the last) are zeros in an output that
+    held NaN before, and the other rows are the bits of the call without padding: output rows shorter and longer than
+    a wave's store, a grid with fewer waves than pairs (1400 tokens), one sort block and several."""
+    experts, k = 96, 3
+    rng = np.random.default_rng(81 + inter + hidden)
+    switch = _switch(packs(80, hidden, inter, experts), hidden, inter, experts, device)
+    inds = np.stack([rng.choice(experts, k, replace=False) for _ in range(tokens)]).astype(np.int32)
+    dead = rng.random(inds.shape) < share
+    padded = np.where(dead, np.where(rng.random(inds.shape) < 0.5, -1, experts), inds).astype(np.int32)
+    x = bf16_device(mo.bf16r(rng.normal(size=(tokens, hidden)).astype(np.float32)), device)
+    whole = grouped_experts(switch, x, torch.tensor(inds, device=device))
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **kw: empty(*a, **kw).fill_(0xff if kw["dtype"] == torch.uint8
+                                                                               else float("nan")))
+    out = grouped_experts(switch, x, torch.tensor(padded, device=device))
+    monkeypatch.undo()
+    torch.cuda.synchronize()
+    mask = torch.tensor(dead, device=device).unsqueeze(-1)
+    assert torch.equal(out.view(torch.int16), torch.where(mask, 0, whole.view(torch.int16)))
+
+
+@pytest.mark.parametrize("hidden,inter,experts,tokens,k", [(1024, 256, 64, 700, 4), (2560, 640, 32, 120, 10)])
+def test_padded_ids_do_not_slow_an_experts_call(device, hidden, inter, experts, tokens, k):
+    """A call all of whose ids name no expert writes its zeros and computes nothing, so it takes no longer than the
+    call with every id valid (half as long where this was written; zeros stored row by row from the sort's own
+    threads took 4 to 25 times as long)."""
+    rng = np.random.default_rng(83)
+    switch = _switch(packs(82, hidden, inter, experts), hidden, inter, experts, device)
+    inds = torch.tensor(np.stack([rng.choice(experts, k, replace=False) for _ in range(tokens)]).astype(np.int32),
+                        device=device)
+    x = bf16_device(rng.normal(size=(tokens, hidden)).astype(np.float32), device)
+
+    def median(ids):
+        times = []
+        for _ in range(25):
+            start, stop = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            start.record()
+            for _ in range(4):
+                grouped_experts(switch, x, ids)
+            stop.record()
+            torch.cuda.synchronize()
+            times.append(start.elapsed_time(stop))
+        return sorted(times)[len(times) // 2]
+
+    none = torch.full_like(inds, -1)
+    valid, padded = median(inds), median(none)
+    print(f"[time] four calls: valid ids {valid * 1e3:.0f} us, no id valid {padded * 1e3:.0f} us", flush=True)
+    assert padded <= 1.25 * valid

@@ -1149,10 +1149,7 @@ static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char
   // of leaving the sorted rows for a copy (700 rows of hidden 1024, 64 experts
   // top-4: 34.8 -> 30.8 us per call)
   const bool scatter = whole_rows && g.mode == 2 && !g.shared && !g.counted;
-  if (scatter) {
-    s.slot_out = static_cast<uint16_t*>(g.output);
-    s.hidden = g.H;
-  }
+  s.by_row = scatter;
   hipError_t e = g.counted ? vm::launch_sort_counted(s, stream) : vm::launch_sort(s, stream);
   if (e != hipSuccess) return hip_fail(e, "sort launch");
 
@@ -1197,7 +1194,11 @@ static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char
   q.shared[1] = vm::ProjPtrs{};
   q.part[0] = 2;
   q.out = scatter ? g.output : ws + w.rows;
-  q.out_row = scatter ? s.pair_row : nullptr;
+  if (scatter) {
+    q.out_row = s.pair_row;
+    q.inds = g.inds;
+    q.pairs = g.T * g.K;
+  }
   q.k_dim = g.I;
   q.n_dim = g.H;
   q.a_stride = g.I;

@@ -1172,7 +1172,7 @@ struct DownB {
   }
 };
 
-template <int QG, int WAVES, int SPB, int MBU>
+template <int QG, int WAVES, int SPB, int MBU, bool SLOTS>
 __device__ __forceinline__ void down_rows_tile(const GroupedLaunch& p, const ProjPtrs& w, uint32_t row0, uint32_t rows,
                                                uint32_t slice0, uint8_t* s_a) {
   constexpr int kThreads = WAVES * 64;
@@ -1197,7 +1197,7 @@ __device__ __forceinline__ void down_rows_tile(const GroupedLaunch& p, const Pro
   uint32_t* s_out = reinterpret_cast<uint32_t*>(s_a + kGroupedRowsDown * kRowBytes + WAVES * 32u * B::kStrip);
   if (tid < MBU * 16) {
     const uint32_t r = row0 + min(tid, rows - 1);
-    s_out[tid] = p.out_row != nullptr ? p.out_row[r] : r;
+    s_out[tid] = SLOTS ? p.out_row[r] : r;
   }
   // columns past N read the last row and are not stored
   const auto column = [&](int s) { return ((slice0 + s) * WAVES + wave) * 16u + bn; };
@@ -1263,7 +1263,26 @@ __device__ __forceinline__ void down_rows_tile(const GroupedLaunch& p, const Pro
   }
 }
 
-template <int QG, int WAVES, int SPB>
+// The output rows of pairs that name no expert are zeros, written by blocks of
+// their own behind those of the tiles: every wave looks at kZeroPairs pairs, its
+// lanes write 16 bytes of a row each.  700 rows of hidden 1024 (64 experts
+// top-4) take 28 us per call with a third of the ids -1 and 23 with all of them
+// (zeroed by the sort's own threads, one row each, 274 and 809).
+constexpr uint32_t kZeroPairs = 8;
+
+__device__ __forceinline__ void zero_rows_without_expert(const GroupedLaunch& p, uint32_t first, uint32_t lane) {
+  const uint32_t i = first + lane;
+  const bool mine = lane < kZeroPairs && i < p.pairs;
+  const uint32_t id = mine ? static_cast<uint32_t>(p.inds[i]) : 0u;
+  for (uint64_t dead = __ballot(mine && id >= p.experts); dead != 0; dead &= dead - 1) {
+    const uint32_t pair = first + static_cast<uint32_t>(__builtin_ctzll(dead));
+    uint4* row = reinterpret_cast<uint4*>(static_cast<uint16_t*>(p.out) + static_cast<size_t>(pair) * p.n_dim);
+    for (uint32_t u = lane; u < p.n_dim / 8; u += 64) row[u] = make_uint4(0, 0, 0, 0);
+  }
+}
+
+// SLOTS: the rows go to the caller's [pair, hidden] output (p.out_row).
+template <int QG, int WAVES, int SPB, bool SLOTS>
 __global__ __launch_bounds__(WAVES * 64, 4) void k_down_rows(GroupedLaunch p) {
   extern __shared__ uint4 s_dyn[];
   uint8_t* s_a = reinterpret_cast<uint8_t*>(s_dyn);
@@ -1274,7 +1293,15 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_down_rows(GroupedLaunch p) {
   const uint32_t lin = blockIdx.x, local = (lin >> 3) / slices, slice0 = (lin >> 3) % slices * SPB;
   const uint32_t count = *p.tile_count, chunk = (count + 7) / 8;
   const uint32_t tile = (lin & 7u) * chunk + local;
-  if (local >= chunk || tile >= count) return;
+  if (local >= chunk || tile >= count) {
+    // the blocks behind the tiles' end up here too; asked for before the tile
+    // count, tile_blocks kept every block waiting (9.4 -> 10.0 us per launch)
+    if (SLOTS && lin >= p.tile_blocks) {
+      const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+      zero_rows_without_expert(p, ((lin - p.tile_blocks) * WAVES + wave) * kZeroPairs, tid & 63u);
+    }
+    return;
+  }
   const uint2 td = p.tiles[tile];
   const uint32_t group = td.x;
   const uint32_t row0 = p.row_off[group] + td.y;
@@ -1293,28 +1320,24 @@ __global__ __launch_bounds__(WAVES * 64, 4) void k_down_rows(GroupedLaunch p) {
     for (uint32_t i = tid; i < rows * cols; i += WAVES * 64) {
       const uint32_t col = slice0 * WAVES * 16 + i % cols;
       const uint32_t r = row0 + i / cols;
-      if (col < N) ActBF16::store(p.out, static_cast<size_t>(p.out_row != nullptr ? p.out_row[r] : r) * N + col, 0.0f);
+      if (col < N) ActBF16::store(p.out, static_cast<size_t>(SLOTS ? p.out_row[r] : r) * N + col, 0.0f);
     }
     return;
   }
-  if (rows > 32) down_rows_tile<QG, WAVES, SPB, 3>(p, w, row0, rows, slice0, s_a);
-  else if (rows > 16) down_rows_tile<QG, WAVES, SPB, 2>(p, w, row0, rows, slice0, s_a);
-  else down_rows_tile<QG, WAVES, SPB, 1>(p, w, row0, rows, slice0, s_a);
+  if (rows > 32) down_rows_tile<QG, WAVES, SPB, 3, SLOTS>(p, w, row0, rows, slice0, s_a);
+  else if (rows > 16) down_rows_tile<QG, WAVES, SPB, 2, SLOTS>(p, w, row0, rows, slice0, s_a);
+  else down_rows_tile<QG, WAVES, SPB, 1, SLOTS>(p, w, row0, rows, slice0, s_a);
 }
 
 // ------------------------------------------------------------------ sort ---
 
 // Pair i got sorted row pos, or names no expert.  Where the down GEMM stores
-// straight into the caller's rows [pair, hidden] (slot_out) the list holds the
-// pair of every row, and the row of a pair without an expert is zeroed here.
+// straight into the caller's rows [pair, hidden] (by_row) the list holds the
+// pair of every row; that kernel also zeroes the rows of pairs without an
+// expert.
 __device__ __forceinline__ void sort_pair(const SortLaunch& p, uint32_t i, uint32_t pos, bool live) {
-  if (p.slot_out == nullptr) {
-    p.pair_row[i] = live ? pos : kNoRow;
-  } else if (live) {
-    p.pair_row[pos] = i;
-  } else {
-    for (uint32_t h = 0; h < p.hidden; ++h) p.slot_out[static_cast<size_t>(i) * p.hidden + h] = 0;
-  }
+  if (!p.by_row) p.pair_row[i] = live ? pos : kNoRow;
+  else if (live) p.pair_row[pos] = i;
 }
 
 // Inclusive scan of one value per thread over a block of 1024 threads.
@@ -1887,10 +1910,10 @@ hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipS
 
 // SPB: column blocks per wave; fewer at the narrow width, whose calls would
 // not fill the chip.
-template <int QG, int SPB>
+template <int QG, int SPB, bool SLOTS>
 hipError_t down_rows_go(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
   constexpr int kWaves = 8;
-  auto kernel = &k_down_rows<QG, kWaves, SPB>;
+  auto kernel = &k_down_rows<QG, kWaves, SPB, SLOTS>;
   constexpr uint32_t lds = kGroupedRowsDown * 4u * QG * kGroup * 2u + kWaves * 32u * DownB<QG>::kStrip +
                            kGroupedRowsDown * 4u;
   static bool attr = false;  // one attribute call per kernel instance
@@ -1901,12 +1924,14 @@ hipError_t down_rows_go(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t 
     attr = true;
   }
   const uint32_t cols = kWaves * 16 * SPB;
-  const dim3 grid(((p.n_dim + cols - 1) / cols) * ((max_tiles + 7) / 8 * 8));
+  GroupedLaunch q = p;
+  q.tile_blocks = ((p.n_dim + cols - 1) / cols) * ((max_tiles + 7) / 8 * 8);
+  const dim3 grid(q.tile_blocks + (SLOTS ? (p.pairs + kWaves * kZeroPairs - 1) / (kWaves * kZeroPairs) : 0u));
   hipEvent_t start = nullptr, stop = nullptr;
   if (timing_events("grouped_down", &start, &stop))
-    hipExtLaunchKernelGGL(kernel, grid, dim3(kWaves * 64), lds, stream, start, stop, 0, p);
+    hipExtLaunchKernelGGL(kernel, grid, dim3(kWaves * 64), lds, stream, start, stop, 0, q);
   else
-    hipLaunchKernelGGL(kernel, grid, dim3(kWaves * 64), lds, stream, p);
+    hipLaunchKernelGGL(kernel, grid, dim3(kWaves * 64), lds, stream, q);
   return hipGetLastError();
 }
 
@@ -1914,9 +1939,10 @@ bool down_rows_supported(uint32_t k_dim) { return k_dim == 256 || k_dim == 640; 
 
 hipError_t launch_down_rows(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
   if (p.a_stride != p.k_dim || p.row_token != nullptr) return hipErrorInvalidValue;
+  const bool slots = p.out_row != nullptr;
   switch (p.k_dim) {
-    case 256: return down_rows_go<2, 2>(p, max_tiles, stream);
-    case 640: return down_rows_go<5, 4>(p, max_tiles, stream);
+    case 256: return slots ? down_rows_go<2, 2, true>(p, max_tiles, stream) : down_rows_go<2, 2, false>(p, max_tiles, stream);
+    case 640: return slots ? down_rows_go<5, 4, true>(p, max_tiles, stream) : down_rows_go<5, 4, false>(p, max_tiles, stream);
     default: return hipErrorInvalidValue;
   }
 }

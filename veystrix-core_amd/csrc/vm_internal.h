@@ -259,7 +259,12 @@ struct GroupedLaunch {
   // counters of the sort that follows the select)
   uint32_t* zero_words;
   uint32_t zero_count;
-  const uint32_t* out_row;     // k_down_rows: output row of every sorted row, or null (the sorted rows)
+  // k_down_rows: output row (pair) of every sorted row, or null (the sorted
+  // rows); with it the pairs' expert ids, whose rows without one are zeroed
+  const uint32_t* out_row;
+  const int32_t* inds;
+  uint32_t pairs;
+  uint32_t tile_blocks;        // blocks of the grid that serve tiles (set by launch_down_rows)
 };
 
 // Router logits of grouped calls as a bf16 GEMM streamed through an LDS ring
@@ -283,10 +288,7 @@ struct SortLaunch {
   uint32_t* status;
   uint32_t tokens, slots, experts, shared_rows;
   uint32_t tile_rows, tile_rows_dn;  // rows per tile of the two lists
-  // not null: pair_row receives the pair of every row instead, and the rows
-  // [pair, hidden] here of pairs without an expert are zeroed
-  uint16_t* slot_out;
-  uint32_t hidden;
+  bool by_row;                 // pair_row receives the pair of every row instead
 };
 
 struct CombineLaunch {
