@@ -1,0 +1,56 @@
+"""What the compiler made of the kernels whose occupancy or ordering the results and timings rely on, from one
+device-only compile to assembly of each source (no GPU needed): registers, scratch and the ordering points that stay
+in the listing as comments."""
+import os
+import re
+import subprocess
+from collections import namedtuple
+
+import pytest
+
+from veymoe import build
+
+Kernel = namedtuple("Kernel", "vgprs scratch wave_barriers")
+_COMPILED = {}
+
+
+def _kernels(source, tmp_path_factory):
+    """Kernel by mangled name for one file of csrc, compiled once."""
+    if source not in _COMPILED:
+        try:
+            hipcc = build.hipcc()
+        except RuntimeError:
+            pytest.skip("hipcc is not installed")
+        listing = tmp_path_factory.mktemp("listing") / "device.s"
+        cmd = [hipcc, *build.HIP_FLAGS, "--cuda-device-only", "-S", os.path.join(build.CSRC, source), "-o", str(listing)]
+        proc = subprocess.run(cmd, capture_output=True, text=True)
+        assert proc.returncode == 0, proc.stderr[-2000:]
+        text = listing.read_text()
+        meta = {m.group(1): m.group(0) for m in re.finditer(r"\.amdhsa_kernel (\S+)\n.*?\.end_amdhsa_kernel", text, re.S)}
+        found = {}
+        for m in re.finditer(r"^(_Z\S+):.*?^\.Lfunc_end\d+:", text, re.M | re.S):
+            if m.group(1) not in meta:
+                continue
+            value = lambda key: int(re.search(rf"\.amdhsa_{key} (\d+)", meta[m.group(1)]).group(1))
+            found[m.group(1)] = Kernel(value("next_free_vgpr"), value("private_segment_fixed_size"),
+                                       m.group(0).count("; wave barrier"))
+        _COMPILED[source] = found
+    return _COMPILED[source]
+
+
+def _instances(kernels, prefix):
+    found = {name: k for name, k in kernels.items() if prefix in name}
+    assert found, f"no kernel matching {prefix}"
+    return found
+
+
+def test_down_rows_keeps_the_order_of_its_strips(tmp_path_factory):
+    """k_down_rows passes each column block's scales through one strip of LDS per wave: stores, then reads by other
+    lanes, then the next block's stores.  Both orders are points the compiler may not move LDS accesses across: with
+    SPB column blocks, 2 SPB - 1 of them in each of the three tile heights' code.  Two blocks of eight waves per CU
+    (four waves per SIMD) take at most 128 registers."""
+    kernels = _instances(_kernels("grouped.hip", tmp_path_factory), "k_down_rowsILi")
+    for name, k in kernels.items():
+        blocks = int(re.search(r"k_down_rowsILi\d+ELi8ELi(\d+)E", name).group(1))
+        assert k.wave_barriers == 3 * (2 * blocks - 1), (name, k)
+        assert k.vgprs <= 128 and k.scratch == 0, (name, k)

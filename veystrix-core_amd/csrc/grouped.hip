@@ -1221,12 +1221,18 @@ __device__ __forceinline__ void down_rows_tile(const GroupedLaunch& p, const Pro
       __builtin_amdgcn_sched_barrier(0);
     }
     const B& bs = b[s & 1];
+    // the strips are read by other lanes of this wave only.  LDS works in order
+    // within a wave, so all it takes is that the compiler keeps that order: the
+    // last block's reads, these stores, this block's reads
+    const auto wave_order = [] {
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+      __builtin_amdgcn_wave_barrier();
+      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    };
+    if (s > 0) wave_order();
     B::put(strip, bs.s, q);
     B::put(strip + 16u * B::kStrip, bs.b, q);
-    // read by other lanes of this wave only: LDS works in order within a wave
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_order();
     f32x4_t acc[MBU];
 #pragma unroll
     for (int mb = 0; mb < MBU; ++mb) acc[mb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
