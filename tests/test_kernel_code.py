@@ -54,3 +54,18 @@ def test_down_rows_keeps_the_order_of_its_strips(tmp_path_factory):
         blocks = int(re.search(r"k_down_rowsILi\d+ELi8ELi(\d+)E", name).group(1))
         assert k.wave_barriers == 3 * (2 * blocks - 1), (name, k)
         assert k.vgprs <= 128 and k.scratch == 0, (name, k)
+
+
+def test_decode_kernels_take_no_scratch(tmp_path_factory):
+    """No decode GEMV has a scratch frame, whatever the compiler keeps in it."""
+    kernels = _kernels("decode.hip", tmp_path_factory)
+    for name, k in {**_instances(kernels, "k_gateupINS_"), **_instances(kernels, "k_downINS_")}.items():
+        assert k.scratch == 0, (name, k)
+
+
+def test_folded_down_runs_two_blocks_per_cu(tmp_path_factory):
+    """The bf16 down kernel of rows a quarter over a power of two: two blocks of twelve waves per CU, six waves per
+    SIMD, take at most 80 registers each."""
+    for name, k in _instances(_kernels("decode.hip", tmp_path_factory), "k_downINS_7ActBF16E").items():
+        if "ELb0ELi4ELi4E" in name:  # no injection, folded, four row groups
+            assert k.vgprs <= 80, (name, k)

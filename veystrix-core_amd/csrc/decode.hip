@@ -219,7 +219,13 @@ __global__ __launch_bounds__(WAVES * 64) void k_gateup(GateUpLaunch p) {
   // stream view serves split-phase routes only and is read where it is used)
   PoolDev pool = p.pool;
   const PoolDev& stream = p.stream;
-  keep_view<0, 6>(pool);
+  if constexpr (FOLD > 0) {
+    // the header goes into the base: with it held too, the instances of 64 lanes
+    // ran out of SGPRs and took a scratch frame
+    if (pool.base != nullptr) pool.base += pool.header;
+    pool.header = 0;
+  }
+  keep_view<0, 6, FOLD == 0>(pool);
   ProjPtrs gate = p.gate, up = p.up;
   keep_proj(gate);
   keep_proj(up);

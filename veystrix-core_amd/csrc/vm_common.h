@@ -332,10 +332,11 @@ __device__ __forceinline__ void keep_proj(ProjPtrs& q) {
 }
 
 // Local SGPR copy of parts [FIRST, FIRST + PARTS) of a pool view (VM_KEEP).
-template <int FIRST, int PARTS>
+// HEADER false: the header is part of the base already.
+template <int FIRST, int PARTS, bool HEADER = true>
 __device__ __forceinline__ void keep_view(PoolDev& v) {
   VM_KEEP(v.base);
-  VM_KEEP(v.header);
+  if constexpr (HEADER) VM_KEEP(v.header);
   VM_KEEP(v.stride);
   VM_KEEP(v.records);
 #pragma unroll
