@@ -420,7 +420,9 @@ int vm_pool_stage(void* pool_base, uint64_t header_size, uint64_t record_stride,
  *     experts, and the down + combine kernel;
  *   2: two launches, the front and one experts grid that hands its gate/up
  *     activations to its down rows through tagged words.
- * All three give the same bits.  -1 queries.  Returns the previous setting.
+ * All three give the same bits; calls of shapes that 1 and 2 have no instance
+ * for run 0 in every mode, as do hidden and intermediate sizes whose rows 0
+ * sums in another order (10, 20, 40 or 80 groups of 32).  -1 queries.  Returns the previous setting.
  * Pipelines 1 and 2 were measured slower than 0 and are compiled only into a
  * library built with -DVM_FUSED_PIPELINES=1; otherwise modes 1 and 2 return
  * VM_EUNSUPPORTED.  No counterpart in the reference: it is for A/B

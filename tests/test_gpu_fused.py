@@ -77,6 +77,23 @@ def test_fused_equals_three_launch_dense(device, spec, layer_id):
     assert_close(host(yf), ref["output"], f"{spec.name} fused decode")
 
 
+@pytest.mark.parametrize("hidden,inter", [(1280, 256), (512, 640), (2560, 640), (320, 320)])
+def test_fused_equals_three_launch_at_folded_widths(device, hidden, inter):
+    """Rows of 10, 20, 40 and 80 groups, whose quarters over the default's GEMVs sum in other lanes: in hidden, in
+    intermediate, in both.  Top-4, so that the experts grid has a wave for every item; a hundred tokens, as two orders
+    of an fp32 sum round to different bf16 values only now and then."""
+    spec = synth.LayerSpec("folded", hidden, inter, 16, 4, inter, 1)
+    seed = hidden + inter
+    layer = assemble.build_layer(spec, seed, device, dense=True)
+    for stream in range(100):
+        x = assemble.tokens_tensor(spec, seed, device, 1, stream=stream)
+        (yf, inf, scf), *others = _both(layer, x)
+        for y3, in3, sc3 in others:
+            _same(inf, in3, "inds")
+            _same(scf, sc3, "scores")
+            _same(yf, y3, (hidden, inter, stream))
+
+
 def test_fused_full_layer_through_the_pool(device):
     """hidden 2048 / inter 512 / 512 experts top-10 + shared, every expert at a
     random slot of a pool behind the slot table (the benchmark's layer)."""

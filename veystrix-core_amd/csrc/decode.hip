@@ -667,12 +667,6 @@ __global__ __launch_bounds__(kBlock) void k_weighted_combine(const void* values,
 
 // ------------------------------------------------------------ dispatch ----
 
-uint32_t next_pow2(uint32_t v) {
-  uint32_t r = 1;
-  while (r < v) r <<= 1;
-  return r;
-}
-
 // One kernel launch of a timing family; with timing on, the start/stop events
 // ride on the dispatch itself.
 template <class... KArgs, class... Args>
@@ -686,18 +680,13 @@ hipError_t launch(const char* family, void (*kernel)(KArgs...), dim3 grid, dim3 
   return hipGetLastError();
 }
 
-// Rows of a power of two of groups and a quarter of it over (hidden 2560: 80 =
-// 64 + 16; inter 640: 20 = 16 + 4): a lane takes one group of each whole row,
-// and the quarters over of four rows make one more load of the whole lane
+// Rows of a quarter over (quarter_over): a lane takes one group of each whole
+// row, and the quarters over of four rows make one more load of the whole lane
 // group.  With lanes for the next power of two, 38 % of them had no group:
 // hidden 2560 / inter 640, one / five / eight tokens 24.6 / 73.0 / 107.5 us per
 // layer, 21.7 / 63.3 / 85.6 folded (20.7 / 57.1 / 76.9 with 32-bit offsets and
 // the shorter unpacking, 20.3 / 52.1 / 70.0 with down's activations in LDS).
 constexpr int kFold = 4;
-bool quarter_over(uint32_t groups) {
-  const uint32_t whole = next_pow2(groups) / 2;
-  return whole >= 8 && whole <= 64 && groups * kFold == whole * (kFold + 1);
-}
 
 template <class A, int LPR, int GI, int U, int FOLD, int WAVES>
 hipError_t gateup_launch(const GateUpLaunch& p, hipStream_t stream) {

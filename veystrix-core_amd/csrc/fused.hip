@@ -25,7 +25,8 @@
 //
 // The arithmetic is the three-launch path's, operation for operation (the
 // same group dots, DPP reduction trees, SwiGLU and combine order), so both
-// give the same bits.
+// give the same bits.  Rows of a quarter over (quarter_over), which that path
+// sums in another order, are left to it.
 
 #include <hip/hip_ext.h>
 #include <hip/hip_runtime.h>
@@ -485,17 +486,11 @@ hipError_t launch(const char* family, void (*kernel)(KArgs...), dim3 grid, dim3 
   return hipGetLastError();
 }
 
-uint32_t pow2_at_least(uint32_t v) {
-  uint32_t r = 1;
-  while (r < v) r <<= 1;
-  return r;
-}
-
 // (lanes per gate/up row, groups per lane) of a hidden size; (0, 0) when the
 // fused kernels have no instance for it
 void gateup_shape(uint32_t hidden, uint32_t& lg, uint32_t& gi) {
   const uint32_t G = hidden / kGroup;
-  lg = G >= 64 ? 64 : pow2_at_least(G);
+  lg = G >= 64 ? 64 : next_pow2(G);
   gi = (G + 63) / 64;
   // hidden sizes above 4096 (four groups per lane) would spill: the
   // three-launch path serves them
@@ -526,7 +521,7 @@ hipError_t experts_go(const FusedLaunch& p0, uint32_t blocks, hipStream_t stream
 template <int LG, int GI>
 hipError_t experts_by_down(const FusedLaunch& p, uint32_t blocks, bool down, hipStream_t stream) {
   if (!down) return experts_go<LG, GI, 4, false>(p, blocks, stream);
-  switch (pow2_at_least(p.inter / kGroup)) {
+  switch (next_pow2(p.inter / kGroup)) {
     case 4: return experts_go<LG, GI, 4, true>(p, blocks, stream);
     case 8: return experts_go<LG, GI, 8, true>(p, blocks, stream);
     case 16: return experts_go<LG, GI, 16, true>(p, blocks, stream);
@@ -540,10 +535,13 @@ hipError_t experts_by_down(const FusedLaunch& p, uint32_t blocks, bool down, hip
 
 bool fused_plan(uint32_t hidden, uint32_t inter, uint32_t slots, uint32_t has_shared, uint32_t experts,
                 uint32_t blocks, FusedLaunch& p) {
+  // the three-launch path sums rows of a quarter over in an order of its own,
+  // and serves them in every mode
+  if (quarter_over(hidden / kGroup) || quarter_over(inter / kGroup)) return false;
   uint32_t lg, gi;
   gateup_shape(hidden, lg, gi);
   const uint32_t GD = inter / kGroup;
-  const uint32_t ld = pow2_at_least(GD);
+  const uint32_t ld = next_pow2(GD);
   if (lg == 0 || ld < 4 || ld > 64 || inter > kFusedMaxInter || slots == 0 || experts == 0 ||
       experts > 64u * kMaxExpertsPerLane || slots + has_shared > kFusedMaxSlots || blocks == 0)
     return false;

@@ -102,6 +102,22 @@ struct DownLaunch {
   uint32_t generic;            // 1: generic combine (products rounded before the slot sum)
 };
 
+// ------------------------------------------------- row shapes of the GEMVs --
+inline uint32_t next_pow2(uint32_t v) {
+  uint32_t r = 1;
+  while (r < v) r <<= 1;
+  return r;
+}
+
+// Rows of a power of two of groups, 8 to 64, and a quarter of it over (hidden
+// 2560: 80 = 64 + 16; inter 640: 20 = 16 + 4).  The decode GEMVs fold the
+// quarters of four rows into one load, so such a row's sum runs in another
+// order than over one lane per group.
+inline bool quarter_over(uint32_t groups) {
+  const uint32_t whole = next_pow2(groups) / 2;
+  return whole >= 8 && whole <= 64 && groups * 4 == whole * 5;
+}
+
 // ---------------------------------------------------- fused decode (T = 1) --
 // The one-token pipelines are built only on request (A/B measurement).
 #ifndef VM_FUSED_PIPELINES
