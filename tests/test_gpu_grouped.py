@@ -506,3 +506,19 @@ def test_padded_ids_do_not_slow_an_experts_call(device, hidden, inter, experts, 
     valid, padded = median(inds), median(none)
     print(f"[time] four calls: valid ids {valid * 1e3:.0f} us, no id valid {padded * 1e3:.0f} us", flush=True)
     assert padded <= 1.25 * valid
+
+
+@pytest.mark.parametrize("hidden,inter", [(384, 512), (384, 256), (256, 384), (256, 640)])
+def test_small_calls_of_one_supported_size_give_the_larger_calls_bits(device, hidden, inter):
+    """The 16-row tile kernels, whose K order is their own, run only where both sizes have an instance: with one of
+    them alone, the rows of a 40-token call have the bits of the same rows in a call of 130."""
+    experts, k = 24, 3
+    rng = np.random.default_rng(85 + hidden + inter)
+    switch = _switch(packs(84, hidden, inter, experts), hidden, inter, experts, device)
+    inds = torch.tensor(np.stack([rng.choice(experts, k, replace=False) for _ in range(130)]).astype(np.int32),
+                        device=device)
+    x = bf16_device(mo.bf16r(rng.normal(size=(130, hidden)).astype(np.float32)), device)
+    small = grouped_experts(switch, x[:40].contiguous(), inds[:40].contiguous())
+    large = grouped_experts(switch, x, inds)
+    torch.cuda.synchronize()
+    assert torch.equal(small.view(torch.int16), large[:40].view(torch.int16))

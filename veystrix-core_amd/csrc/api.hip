@@ -526,7 +526,7 @@ struct GroupedWs {
   uint64_t logits, sig, inds, scores, row_off, tiles, tile_count, tiles_dn, tile_count_dn, sort_counts,
       sort_cursors, row_token, pair_row, act, rows, total;
   uint32_t rows_total, groups, max_tiles, max_tiles_dn, tile_rows, tile_rows_dn;
-  bool small, small_dn;  // 16-row tile kernels (k_rows) for gate/up and down
+  bool small;  // 16-row tile kernels (k_rows)
 };
 
 // Calls of up to this many tokens run the 16-row tile kernels, whose blocks
@@ -542,12 +542,11 @@ constexpr uint32_t kRowsMaxTokens = 64;
 #ifndef VM_ROUTER_RING
 #define VM_ROUTER_RING 1
 #endif
-static bool small_gateup(uint32_t T, uint32_t H) {
-  return VM_ROWS_PATH && T <= kRowsMaxTokens && vm::rows_gateup_supported(H);
-}
-
-static bool small_down(uint32_t T, uint32_t I) {
-  return VM_ROWS_PATH && T <= kRowsMaxTokens && vm::rows_down_supported(I);
+// Only where both sizes have an instance: with the one that has, alone, hidden
+// 2560 / inter 512 (512 experts top-10) took 237 us at 64 rows where the chunked
+// GEMM takes 221, and hidden 1536 / inter 256 (128 experts top-8) 47.8 and 46.0.
+static bool small_grouped(uint32_t T, uint32_t H, uint32_t I) {
+  return VM_ROWS_PATH && T <= kRowsMaxTokens && vm::rows_supported(H) && vm::rows_supported(I);
 }
 
 // Rows per gate/up tile of a chunked-GEMM call: tall tiles when the routed
@@ -569,14 +568,13 @@ static uint32_t down_tile_rows(uint32_t T, uint32_t K, uint32_t I, uint32_t E) {
   return tall ? vm::kGroupedRowsTall : vm::kGroupedRowsDown;
 }
 
-static GroupedWs grouped_ws_of(uint32_t T, uint32_t K, uint32_t H, uint32_t I, uint32_t E, bool shared, bool small_dn) {
+static GroupedWs grouped_ws(uint32_t T, uint32_t K, uint32_t H, uint32_t I, uint32_t E, bool shared) {
   GroupedWs w{};
   w.rows_total = T * K + (shared ? T : 0);
   w.groups = E + (shared ? 1 : 0);
-  w.small = small_gateup(T, H);
-  w.small_dn = small_dn;
+  w.small = small_grouped(T, H, I);
   w.tile_rows = w.small ? vm::kRowsTile : gateup_tile_rows(T, K, H, E);
-  w.tile_rows_dn = w.small_dn ? vm::kRowsTile : down_tile_rows(T, K, I, E);
+  w.tile_rows_dn = w.small ? vm::kRowsTile : down_tile_rows(T, K, I, E);
   w.max_tiles = vm::grouped_max_tiles(w.rows_total, w.groups, w.tile_rows);
   w.max_tiles_dn = vm::grouped_max_tiles(w.rows_total, w.groups, w.tile_rows_dn);
   uint64_t o = kAlign;
@@ -604,16 +602,6 @@ static GroupedWs grouped_ws_of(uint32_t T, uint32_t K, uint32_t H, uint32_t I, u
   w.rows = take(uint64_t(w.rows_total) * H * 2);
   w.total = o;
   return w;
-}
-
-// The tile list of 16-row down tiles is a little longer: a call that fits the
-// static scratch without them keeps fitting it.
-static GroupedWs grouped_ws(uint32_t T, uint32_t K, uint32_t H, uint32_t I, uint32_t E, bool shared) {
-  const bool small_dn = small_down(T, I);
-  const GroupedWs w = grouped_ws_of(T, K, H, I, E, shared, small_dn);
-  if (!small_dn || w.total <= VM_STATIC_SCRATCH_BYTES) return w;
-  const GroupedWs chunked = grouped_ws_of(T, K, H, I, E, shared, false);
-  return chunked.total <= VM_STATIC_SCRATCH_BYTES ? chunked : w;
 }
 
 static bool use_grouped(uint32_t T, uint32_t dtype) { return T > VM_LAYER_MAX_TOKENS && dtype == VM_BF16; }
@@ -1144,7 +1132,7 @@ static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char
   s.shared_rows = g.shared ? g.T : 0;
   s.tile_rows = w.tile_rows;
   s.tile_rows_dn = w.tile_rows_dn;
-  const bool whole_rows = !w.small_dn && w.tile_rows_dn == vm::kGroupedRowsDown && vm::down_rows_supported(g.I);
+  const bool whole_rows = !w.small && w.tile_rows_dn == vm::kGroupedRowsDown && vm::down_rows_supported(g.I);
   // one output row per token and slot: k_down_rows stores there itself instead
   // of leaving the sorted rows for a copy (700 rows of hidden 1024, 64 experts
   // top-4: 34.8 -> 30.8 us per call)
@@ -1204,10 +1192,10 @@ static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char
   q.a_stride = g.I;
   q.a_rows = g.T * g.K + (g.shared ? g.T : 0);
   q.weights_once = uint64_t(g.T) * g.K <= uint64_t(g.E) * vm::kGroupedRowsDown;
-  q.tile_rows = w.small_dn || w.tile_rows_dn == vm::kGroupedRowsDown ? 0u : w.tile_rows_dn;
+  q.tile_rows = w.small || w.tile_rows_dn == vm::kGroupedRowsDown ? 0u : w.tile_rows_dn;
   q.tiles = s.tiles_dn;
   q.tile_count = s.tile_count_dn;
-  e = w.small_dn ? vm::launch_rows(vm::kEpiRows, q, w.max_tiles_dn, stream)
+  e = w.small ? vm::launch_rows(vm::kEpiRows, q, w.max_tiles_dn, stream)
       : whole_rows ? vm::launch_down_rows(q, w.max_tiles_dn, stream)
                    : vm::launch_grouped(vm::kEpiRows, q, w.max_tiles_dn, stream);
   if (e != hipSuccess) return hip_fail(e, "grouped down launch");

@@ -864,44 +864,30 @@ __device__ __forceinline__ void grouped_block(const GroupedLaunch& p, uint32_t l
 // K order: lane quarter q = lane / 16 owns the contiguous quarter of the
 // groups [q G/4, (q + 1) G/4); MFMA step j feeds packed word j % 4 of the
 // quarter's group j / 4.  So a lane's scales and biases for the whole K are
-// G/4 contiguous bf16 values (loaded once per tile with wide loads: 2-byte
+// 2 KCH contiguous bf16 values (loaded once per tile with wide loads: 2-byte
 // loads per lane and chunk had cost more than the weights), and its weights
-// of a chunk (two groups, one in the last chunk of an odd quarter) are 32
-// contiguous bytes.  The fp32 sums over K run
+// of a chunk (two groups) are 32 contiguous bytes.  The fp32 sums over K run
 // in a different order from the chunked GEMM, within the same tolerance.
 // A row r stores its 16-byte unit u at (u & ~15) | ((u ^ rows_swz(r, q)) & 15):
 // at step j the 64 lanes (16 rows x 4 quarters) read units q G/4*4 + j, which
-// this spreads over all 16 bank groups, four lanes each.  Where a quarter is
-// not whole blocks (or halves) of 16 units (K = 640) units of two quarters
-// share a block, so the XOR is by the row alone there.
+// this spreads over all 16 bank groups, four lanes each.
 constexpr int kRowsDepth = 3;  // chunks of weight loads in flight per wave
+constexpr int kRowsCG = 8;     // 32-input groups per k_rows chunk (K = 256 KCH)
 
 __device__ __forceinline__ constexpr uint32_t rows_swz(uint32_t r, uint32_t q) { return (r ^ (q << 2)) & 15u; }
 
-// VALS consecutive bf16 values in pairs, in the widest loads: from a 4-byte
-// aligned address, or for an odd count from a 2-byte aligned one (four bytes at
-// a time from any address, and the last value by itself, so that nothing past
-// it is read).
-typedef uint32_t u32_align2 __attribute__((aligned(2)));
-template <int VALS, int N = (VALS + 1) / 2>
-__device__ __forceinline__ void ldg_pairs(const uint8_t* src, uint32_t (&out)[N]) {
-  if constexpr (VALS % 2 != 0) {
-#pragma unroll
-    for (int i = 0; i < N - 1; ++i)
-      out[i] = *(const __attribute__((address_space(1))) u32_align2*)(src + 4 * i);
-    out[N - 1] = ldg_u16(src + 4 * (N - 1));
-  } else if constexpr (N % 4 == 0) {
+// n consecutive dwords from a 4-byte aligned address, in the widest loads
+template <int N>
+__device__ __forceinline__ void ldg_dwords(const uint8_t* src, uint32_t (&out)[N]) {
+  if constexpr (N % 4 == 0) {
 #pragma unroll
     for (int i = 0; i < N; i += 4) {
       const uint4 v = ldg16(src + 4 * i);
       out[i] = v.x; out[i + 1] = v.y; out[i + 2] = v.z; out[i + 3] = v.w;
     }
-  } else if constexpr (N % 2 == 0) {
-#pragma unroll
-    for (int i = 0; i < N; i += 2) {
-      const uint2 v = *reinterpret_cast<const uint2*>(src + 4 * i);
-      out[i] = v.x; out[i + 1] = v.y;
-    }
+  } else if constexpr (N == 2) {
+    const uint2 v = *reinterpret_cast<const uint2*>(src);
+    out[0] = v.x; out[1] = v.y;
   } else {
 #pragma unroll
     for (int i = 0; i < N; ++i) out[i] = *reinterpret_cast<const uint32_t*>(src + 4 * i);
@@ -909,21 +895,20 @@ __device__ __forceinline__ void ldg_pairs(const uint8_t* src, uint32_t (&out)[N]
 }
 
 // One (tile, column slice) item of block-uniform index `item`; false when the
-// item is past the live tiles.  QG: K = 128 QG (the instance is picked per
+// item is past the live tiles.  KCH: K = 256 KCH (the instance is picked per
 // K), so the kernel is straight-line and every wait counts exactly the loads
 // it needs.  Load order: the tile's row indices (lanes 0-15), its A rows, the
 // lane's scales and biases, the first kRowsDepth chunks of weights; the A
 // rows go to LDS as they arrive, with the weight loads still in flight.
-template <int EPI, int WAVES, int PROJ, int QG>
+template <int EPI, int WAVES, int PROJ, int KCH>
 __device__ __forceinline__ bool rows_item(const GroupedLaunch& p, uint32_t item, uint8_t* s_a, PhaseTrace& tr) {
   constexpr int kThreads = WAVES * 64;
   constexpr int kCols = WAVES * 16;
-  constexpr int kQG = QG;                          // groups per lane quarter
-  constexpr int kG = 4 * QG;                       // groups of K
-  constexpr int KCH = (QG + 1) / 2;                // chunks
-  constexpr uint32_t kSwzQ = QG % 4 == 0 || QG == 2 ? 1 : 0;  // the quarter is part of the swizzle
+  constexpr int kG = KCH * kRowsCG;                // groups of K
+  constexpr int kQG = kG / 4;                      // groups per lane quarter (2 KCH)
   constexpr int kUnits = kG * 4;                   // 16-byte A units per row
   constexpr int kRowBytes = kUnits * 16;
+  static_assert((16 * kUnits) % kThreads == 0, "whole A units per thread");
   const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
   const uint32_t K = p.k_dim, N = p.n_dim;
 
@@ -984,8 +969,8 @@ __device__ __forceinline__ bool rows_item(const GroupedLaunch& p, uint32_t item,
 #pragma unroll
     for (int pj = 0; pj < PROJ; ++pj) {
       const size_t m = (static_cast<size_t>(col_ld) * kG + g_lane) * 2u;
-      ldg_pairs<QG>(reinterpret_cast<const uint8_t*>(w[pj].s) + m, sv[pj]);
-      ldg_pairs<QG>(reinterpret_cast<const uint8_t*>(w[pj].b) + m, bv[pj]);
+      ldg_dwords<KCH>(reinterpret_cast<const uint8_t*>(w[pj].s) + m, sv[pj]);
+      ldg_dwords<KCH>(reinterpret_cast<const uint8_t*>(w[pj].b) + m, bv[pj]);
     }
     // keep the prefetch here and in chunk order: the scheduler otherwise sinks
     // every chunk's loads to just before their first use, or mixes the chunks,
@@ -996,15 +981,14 @@ __device__ __forceinline__ bool rows_item(const GroupedLaunch& p, uint32_t item,
 #pragma unroll
       for (int pj = 0; pj < PROJ; ++pj) {
         bw[d][pj][0] = ldg16(wl[pj] + d * 32u);
-        if (2 * d + 1 < kQG) bw[d][pj][1] = ldg16(wl[pj] + d * 32u + 16u);
+        bw[d][pj][1] = ldg16(wl[pj] + d * 32u + 16u);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
 
   // A rows: R rows of the tile are loaded (R = 4, 8 or 16, the least that
-  // holds it and keeps most threads busy; threads past the last unit repeat
-  // it); LDS rows past R keep stale
+  // holds it and gives every thread whole units); LDS rows past R keep stale
   // data, which only reaches MFMA output rows that are not stored (an output
   // row depends on its own A row only).  Unit it = j * threads + tid -> (row
   // it / kUnits, unit it % kUnits).  The loads are unconditional (branches
@@ -1013,18 +997,14 @@ __device__ __forceinline__ bool rows_item(const GroupedLaunch& p, uint32_t item,
   const bool gather = p.row_token != nullptr;
   auto stage = [&](auto rows_class) {
     constexpr int R = decltype(rows_class)::value;
-    constexpr int kIt = (R * kUnits + kThreads - 1) / kThreads;
-    const auto unit = [&](int j) {
-      const uint32_t i = j * kThreads + tid;
-      return (R * kUnits) % kThreads == 0 ? i : min(i, static_cast<uint32_t>(R * kUnits - 1));
-    };
+    constexpr int kIt = R * kUnits / kThreads;
     uint4 av[kIt];
 #pragma unroll
     for (int j = 0; j < kIt; ++j) {
-      const uint32_t it = unit(j);
+      const uint32_t it = j * kThreads + tid;
       const uint32_t r = min(it / kUnits, rows - 1), u = it % kUnits;
       uint32_t arow;
-      if constexpr (kUnits % 64 == 0 && (R * kUnits) % kThreads == 0) {  // r is wave-uniform
+      if constexpr (kUnits % 64 == 0) {  // r is wave-uniform
         arow = gather ? __builtin_amdgcn_readlane(my_row, __builtin_amdgcn_readfirstlane(r)) : row0 + r;
       } else {
         arow = gather ? __shfl(my_row, static_cast<int>(r), 64) : row0 + r;
@@ -1035,17 +1015,17 @@ __device__ __forceinline__ bool rows_item(const GroupedLaunch& p, uint32_t item,
     if (p.trace != nullptr) tr.mark(2);
 #pragma unroll
     for (int j = 0; j < kIt; ++j) {
-      const uint32_t it = unit(j);
+      const uint32_t it = j * kThreads + tid;
       const uint32_t r = it / kUnits, u = it % kUnits;
       const uint4 x = av[j];
       const uint4 pp = kNatural ? x
                                 : make_uint4((x.x & 0xffffu) | (x.z << 16), (x.x >> 16) | (x.z & 0xffff0000u),
                                              (x.y & 0xffffu) | (x.w << 16), (x.y >> 16) | (x.w & 0xffff0000u));
-      const uint32_t phys = (u & ~15u) | ((u ^ rows_swz(r, kSwzQ * (u / (kQG * 4)))) & 15u);
+      const uint32_t phys = (u & ~15u) | ((u ^ rows_swz(r, u / (kQG * 4))) & 15u);
       *reinterpret_cast<uint4*>(s_a + r * kRowBytes + phys * 16u) = pp;
     }
   };
-  constexpr bool kR4 = 8 * kUnits > kThreads, kR8 = 16 * kUnits > kThreads;
+  constexpr bool kR4 = (4 * kUnits) % kThreads == 0, kR8 = (8 * kUnits) % kThreads == 0;
   if (kR4 && rows <= 4) stage(std::integral_constant<int, kR4 ? 4 : 16>{});
   else if (kR8 && rows <= 8) stage(std::integral_constant<int, kR8 ? 8 : 16>{});
   else stage(std::integral_constant<int, 16>{});
@@ -1058,7 +1038,7 @@ __device__ __forceinline__ bool rows_item(const GroupedLaunch& p, uint32_t item,
   const uint32_t magic = f16_magic();
   const uint32_t am = lane & 15u;
   const uint8_t* a_lane = s_a + am * kRowBytes;
-  const uint32_t a_sw = rows_swz(am, kSwzQ * q);
+  const uint32_t a_sw = rows_swz(am, q);
   const uint32_t u_lane = q * kQG * 4;             // the lane's first A unit
 #pragma unroll
   for (int c = 0; c < KCH; ++c) {
@@ -1066,7 +1046,6 @@ __device__ __forceinline__ bool rows_item(const GroupedLaunch& p, uint32_t item,
 #pragma unroll
     for (int st = 0; st < 8; ++st) {
       const int gi = 2 * c + (st >> 2);            // group of the lane's quarter
-      if (gi >= kQG) break;
       const uint32_t u = u_lane + gi * 4 + (st & 3);
       const uint32_t phys = (u & ~15u) | ((u ^ a_sw) & 15u);
       const bf16x8_t aop = __builtin_bit_cast(bf16x8_t, *reinterpret_cast<const uint4*>(a_lane + phys * 16u));
@@ -1087,7 +1066,7 @@ __device__ __forceinline__ bool rows_item(const GroupedLaunch& p, uint32_t item,
 #pragma unroll
       for (int pj = 0; pj < PROJ; ++pj) {
         bw[d][pj][0] = ldg16(wl[pj] + (c + kDepth) * 32u);
-        if (2 * (c + kDepth) + 1 < kQG) bw[d][pj][1] = ldg16(wl[pj] + (c + kDepth) * 32u + 16u);
+        bw[d][pj][1] = ldg16(wl[pj] + (c + kDepth) * 32u + 16u);
       }
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -1113,14 +1092,14 @@ __device__ __forceinline__ bool rows_item(const GroupedLaunch& p, uint32_t item,
 // One item per block over the bound of the live tiles (blocks past them exit).
 // A loop of items per block kept loop-invariant arguments live and took the
 // registers of a second block per CU.
-template <int EPI, int WAVES, int PROJ, int QG>
+template <int EPI, int WAVES, int PROJ, int KCH>
 __global__ __launch_bounds__(WAVES * 64) void k_rows(GroupedLaunch p) {
   static_assert(EPI == kEpiSwiglu || EPI == kEpiRows, "Q4 epilogues only");
   extern __shared__ uint4 s_dyn[];
   uint8_t* s_a = reinterpret_cast<uint8_t*>(s_dyn);
   PhaseTrace tr;
   if (p.trace != nullptr) tr.mark(0);
-  const bool live = rows_item<EPI, WAVES, PROJ, QG>(p, blockIdx.x, s_a, tr);
+  const bool live = rows_item<EPI, WAVES, PROJ, KCH>(p, blockIdx.x, s_a, tr);
   if (p.trace != nullptr && threadIdx.x == 0) {
     tr.mark(5);
     tr.t[7] = live ? 1u : 0u;
@@ -1846,27 +1825,23 @@ hipError_t launch_grouped(int epi, const GroupedLaunch& p, uint32_t max_tiles, h
   }
 }
 
-// The k_rows instances: K of 256, 512, 1024, 2048 or 4096 exactly, for down
-// also 640 (their strides are compile-time; the A rows of a 16-row tile take 8
-// to 128 KiB of LDS).  Other K take the chunked GEMM, as does gate/up at 2560:
-// 80 KiB of rows and 219 VGPRs, 42.1 us against the chunked GEMM's 37.0 at 24
-// rows (down at 640: 20.4 against 24.9).
+// The k_rows instances: K of 256, 512, 1024, 2048 or 4096 exactly (their
+// strides are compile-time; the A rows of a 16-row tile take 8 to 128 KiB of
+// LDS).  Other K take the chunked GEMM.
 constexpr uint32_t kRowsMaxK = 4096;
 
 bool down_tall_supported(uint32_t k_dim) {
   return (k_dim / kGroup) % kCG == 0 || half_tail(k_dim / kGroup);
 }
 
-bool rows_gateup_supported(uint32_t k_dim) {
+bool rows_supported(uint32_t k_dim) {
   return k_dim == 256 || k_dim == 512 || k_dim == 1024 || k_dim == 2048 || k_dim == kRowsMaxK;
 }
 
-bool rows_down_supported(uint32_t k_dim) { return rows_gateup_supported(k_dim) || k_dim == 640; }
-
-template <int EPI, int WAVES, int PROJ, int QG>
+template <int EPI, int WAVES, int PROJ, int KCH>
 hipError_t rows_go_k(const char* family, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
-  auto kernel = &k_rows<EPI, WAVES, PROJ, QG>;
-  constexpr uint32_t lds = 16u * 4u * QG * kGroup * 2u;
+  auto kernel = &k_rows<EPI, WAVES, PROJ, KCH>;
+  constexpr uint32_t lds = 16u * KCH * kRowsCG * kGroup * 2u;
   static bool attr = false;  // one attribute call per kernel instance
   if (!attr) {
     hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
@@ -1896,19 +1871,17 @@ hipError_t rows_go_k(const char* family, const GroupedLaunch& p, uint32_t max_ti
 template <int EPI, int WAVES, int PROJ>
 hipError_t rows_go(const char* family, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
   switch (p.k_dim) {
-    case 256: return rows_go_k<EPI, WAVES, PROJ, 2>(family, p, max_tiles, stream);
-    case 512: return rows_go_k<EPI, WAVES, PROJ, 4>(family, p, max_tiles, stream);
-    case 640:
-      if constexpr (EPI == kEpiRows) return rows_go_k<EPI, WAVES, PROJ, 5>(family, p, max_tiles, stream);
-      return hipErrorInvalidValue;
-    case 1024: return rows_go_k<EPI, WAVES, PROJ, 8>(family, p, max_tiles, stream);
-    case 2048: return rows_go_k<EPI, WAVES, PROJ, 16>(family, p, max_tiles, stream);
-    case 4096: return rows_go_k<EPI, WAVES, PROJ, 32>(family, p, max_tiles, stream);
+    case 256: return rows_go_k<EPI, WAVES, PROJ, 1>(family, p, max_tiles, stream);
+    case 512: return rows_go_k<EPI, WAVES, PROJ, 2>(family, p, max_tiles, stream);
+    case 1024: return rows_go_k<EPI, WAVES, PROJ, 4>(family, p, max_tiles, stream);
+    case 2048: return rows_go_k<EPI, WAVES, PROJ, 8>(family, p, max_tiles, stream);
+    case 4096: return rows_go_k<EPI, WAVES, PROJ, 16>(family, p, max_tiles, stream);
     default: return hipErrorInvalidValue;
   }
 }
 
 hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
+  if (!rows_supported(p.k_dim)) return hipErrorInvalidValue;
   if (epi == kEpiSwiglu) return rows_go<kEpiSwiglu, VM_ROWS_GU_WAVES, 2>("grouped_gateup", p, max_tiles, stream);
   if (epi == kEpiRows) return rows_go<kEpiRows, VM_ROWS_DN_WAVES, 1>("grouped_down", p, max_tiles, stream);
   return hipErrorInvalidValue;

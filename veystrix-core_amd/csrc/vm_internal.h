@@ -330,8 +330,7 @@ hipError_t launch_grouped(int epi, const GroupedLaunch& p, uint32_t max_tiles, h
 constexpr int kRowsTile = 16;
 // The down GEMM's staged-weight instances (and so its tall tiles) take this K.
 bool down_tall_supported(uint32_t k_dim);
-bool rows_gateup_supported(uint32_t k_dim);
-bool rows_down_supported(uint32_t k_dim);
+bool rows_supported(uint32_t k_dim);
 hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream);
 // The down GEMM over tiles of up to kGroupedRowsDown rows with whole A rows in
 // LDS (k_down_rows).
