@@ -522,3 +522,26 @@ def test_small_calls_of_one_supported_size_give_the_larger_calls_bits(device, hi
     large = grouped_experts(switch, x, inds)
     torch.cuda.synchronize()
     assert torch.equal(small.view(torch.int16), large[:40].view(torch.int16))
+
+
+@pytest.mark.parametrize("inter", [384, 640, 896])
+@pytest.mark.parametrize("hidden", [1088, 2080])
+def test_down_gemm_of_whole_rows_at_half_chunks_over(device, hidden, inter):
+    """Every instance of k_down_rows whose K has half a chunk over, with two column blocks per wave (hidden 1088) and
+    four (2080), both ending inside a block: the bits of the chunked GEMM's 96-row tiles, which a call of 500 tokens
+    takes, and the oracle's values.  Calls of 20 and 150 tokens; two thirds of the rows go to the last expert."""
+    experts, k, more = 24, 3, 500
+    np_packs = packs(86, hidden, inter, experts)
+    rng = np.random.default_rng(87 + inter + hidden)
+    inds = np.stack([rng.choice(experts - 1, k, replace=False) for _ in range(more)]).astype(np.int32)
+    inds[:100, 0] = experts - 1
+    x_np = mo.bf16r(rng.normal(size=(more, hidden)).astype(np.float32))
+    switch = _switch(np_packs, hidden, inter, experts, device)
+    x, i = bf16_device(x_np, device), torch.tensor(inds, device=device)
+    tall = grouped_experts(switch, x, i)
+    for tokens in (20, 150):
+        out = grouped_experts(switch, x[:tokens].contiguous(), i[:tokens].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), tall[:tokens].view(torch.int16)), tokens
+    _, _, _, d_out, _ = mo.execute(x_np[:20], inds[:20], np_packs, "bf16", qmm=True)
+    _close_qmm(host(tall[:20]), d_out, f"hidden {hidden}, inter {inter}")

@@ -1109,19 +1109,17 @@ __global__ __launch_bounds__(WAVES * 64) void k_rows(GroupedLaunch p) {
 
 // ------------------------------------------------- down GEMM, whole rows ---
 
-// The down GEMM of tiles of up to 48 rows at intermediate sizes of up to 640:
-// the block stages its tile's A rows over the whole K in LDS once, as k_rows
+// The down GEMM of tiles of up to 48 rows at the intermediate sizes of
+// down_rows_supported: the block stages its tile's A rows over the whole K in LDS once, as k_rows
 // does, and every wave streams the weights of SPB column blocks of 16 straight
 // into its MFMA lanes, the next block's loads in flight while one is
 // multiplied, with no barrier after the staging.  The chunked GEMM passes the
-// weights through LDS, two barriers per chunk and a load latency that two or
-// three chunks of K hardly cover; here a dequantised operand feeds as many
-// MFMAs and nothing but the wave's own loads is waited for.  Bound by HBM:
-// hidden 2560 / inter 640, 512 experts top-10, 333 / 1000 / 1999 / 2400 rows:
-// 450 / 504 / 599 / 669 us per call chunked, 402 / 456 / 549 / 607 so (16-row
-// tiles at 333 rows: 416); hidden 1024 / inter 256, 64 experts top-4, 333 rows:
-// 41.8 and 38.8.  At inter 512, two whole chunks, it is the slower one (1999
-// rows 352 and 363 us).
+// weights through LDS, two barriers per chunk and a load latency that a chunk
+// or a few hardly cover; here a dequantised operand feeds as many MFMAs and
+// nothing but the wave's own loads is waited for.  Bound by HBM: hidden 2560 /
+// inter 640, 512 experts top-10, 333 / 1000 / 1999 / 2400 rows: 450 / 504 / 599
+// / 669 us per call chunked, 402 / 456 / 549 / 607 so; hidden 1024 / inter 256,
+// 64 experts top-4, 333 rows: 41.8 and 38.8.
 //
 // K order is the chunked GEMM's: MFMA step (g, i) feeds k block kb from group
 // 4 g + kb, packed word i, so both give the same bits and a row's result does
@@ -1887,10 +1885,22 @@ hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipS
   return hipErrorInvalidValue;
 }
 
-// SPB: column blocks per wave; fewer at the narrow width, whose calls would
-// not fill the chip.
+// k_down_rows takes K of one chunk, and of half a chunk over whole ones up to
+// 896 (102 KB of LDS there, one block per CU).  Where the chunked GEMM runs
+// whole chunks, two and more, it is the better one: per call, ten of 512
+// experts, 1000 rows, hidden 2048 / inter 512 291 us chunked and 305 so, 2560 /
+// 768 531 and 549, but 2560 / 384 334 and 315, 2560 / 896 669 and 645.  Calls of
+// few blocks gain too (hidden 1024, four of 64 experts, 24 rows: inter 384 39.4
+// and 35.0, inter 896 55.3 and 48.4).
+constexpr uint32_t kDownRowsGroups = 28;
+// Column blocks per wave (SPB): four from hidden 2048 up (2560 / 640, 1999 rows:
+// 551 us per call with two, 539 with four), two below, where four leave the chip
+// idle (1024 / 640, four of 64 experts, 400 rows: 57.3 with four, 51.4 with two)
+// and at K = 256.
+constexpr uint32_t kDownRowsWide = 2048;
+
 template <int QG, int SPB, bool SLOTS>
-hipError_t down_rows_go(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
+hipError_t down_rows_go_k(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
   constexpr int kWaves = 8;
   auto kernel = &k_down_rows<QG, kWaves, SPB, SLOTS>;
   constexpr uint32_t lds = kGroupedRowsDown * 4u * QG * kGroup * 2u + kWaves * 32u * DownB<QG>::kStrip +
@@ -1914,14 +1924,28 @@ hipError_t down_rows_go(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t 
   return hipGetLastError();
 }
 
-bool down_rows_supported(uint32_t k_dim) { return k_dim == 256 || k_dim == 640; }
+bool down_rows_supported(uint32_t k_dim) {
+  const uint32_t groups = k_dim / kGroup;
+  return groups == kCG || (half_tail(groups) && groups <= kDownRowsGroups);
+}
+
+template <int QG>
+hipError_t down_rows_go(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
+  const bool slots = p.out_row != nullptr;
+  if constexpr (QG > 2) {
+    if (p.n_dim >= kDownRowsWide)
+      return slots ? down_rows_go_k<QG, 4, true>(p, max_tiles, stream) : down_rows_go_k<QG, 4, false>(p, max_tiles, stream);
+  }
+  return slots ? down_rows_go_k<QG, 2, true>(p, max_tiles, stream) : down_rows_go_k<QG, 2, false>(p, max_tiles, stream);
+}
 
 hipError_t launch_down_rows(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
-  if (p.a_stride != p.k_dim || p.row_token != nullptr) return hipErrorInvalidValue;
-  const bool slots = p.out_row != nullptr;
-  switch (p.k_dim) {
-    case 256: return slots ? down_rows_go<2, 2, true>(p, max_tiles, stream) : down_rows_go<2, 2, false>(p, max_tiles, stream);
-    case 640: return slots ? down_rows_go<5, 4, true>(p, max_tiles, stream) : down_rows_go<5, 4, false>(p, max_tiles, stream);
+  if (p.a_stride != p.k_dim || p.row_token != nullptr || !down_rows_supported(p.k_dim)) return hipErrorInvalidValue;
+  switch (p.k_dim / kGroup) {
+    case 8: return down_rows_go<2>(p, max_tiles, stream);
+    case 12: return down_rows_go<3>(p, max_tiles, stream);
+    case 20: return down_rows_go<5>(p, max_tiles, stream);
+    case 28: return down_rows_go<7>(p, max_tiles, stream);
     default: return hipErrorInvalidValue;
   }
 }
