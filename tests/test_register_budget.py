@@ -3,11 +3,11 @@ resource report (no GPU needed).
 
 The occupancy these kernels are tuned for is set by their registers as much
 as by their LDS:
-* the down GEMM (`k_grouped<1, 8, 2, 1, false, *, 48>`) runs two 8-wave blocks
+* the down GEMM (`k_grouped<1, 8, 2, 1, false, *, *, 48>`) runs two 8-wave blocks
   per CU, four waves per SIMD, so its VGPRs + AGPRs must stay at or below 128
   of the SIMD's 512 per lane (its tall 96-row tiles run one block per CU:
   at most 256);
-* the gate/up GEMM with 64-row tiles (`k_grouped<0, 4, 1, 2, false, *, 64>`)
+* the gate/up GEMM with 64-row tiles (`k_grouped<0, 4, 1, 2, false, *, *, 64>`)
   runs three 4-wave blocks per CU, three waves per SIMD: at most 168 (512 / 3
   in the allocation granule of 8); with the tall 96-row tiles of calls of many
   rows per expert, two blocks per CU: at most 256.
@@ -66,7 +66,7 @@ def _instances(kernels, prefix):
 
 def test_grouped_gemm_register_budgets(kernels):
     # template arguments: EPI, waves, column blocks per wave, projections, tail
-    # chunk, non-temporal weights, tile rows
+    # chunk, non-temporal weights, half a chunk over, tile rows
     # down: 8 waves, 2 column blocks per wave, 1 projection, no tail chunk;
     # 48-row tiles two blocks per CU, the tall 96-row tiles (88 KB of LDS) one
     for name, r in _instances(kernels, "k_groupedILi1ELi8ELi2ELi1ELb0ELb").items():

@@ -100,11 +100,13 @@ constexpr int kWColBytes = kCG * 16;  // LDS bytes per staged weight row chunk (
 // K of half a chunk over, after at least one whole chunk (K = 640: 8 + 8 + 4
 // groups; HALF instances): the last chunk is loaded from the row's last eight
 // groups, all of them inside the row, and only its upper half's MFMA steps
-// run, so rows, weights and scales are staged as in a whole chunk.  Any other
-// remainder (TAIL instances) has its last chunk's loads clamped and its lanes
-// fetch their own weights and 2-byte scales: at hidden 2560 / inter 640 those
-// took the 1999-row call 641 us where these take 596, and 333 rows 505 and
-// 449.  Same products in the same order: the same bits.
+// run, so rows, weights and scales are staged as in a whole chunk.  They serve
+// the down GEMM's tall tiles, and its usual ones above the sizes of
+// k_down_rows.  Any other remainder (TAIL instances) has its last chunk's loads
+// clamped and its lanes fetch their own weights and 2-byte scales: hidden 2048 /
+// inter 1152, eight of 256 experts, 250 / 1000 rows take 344 / 385 us per call
+// with those, 290 / 349 with these.  Same products in the same order: the same
+// bits.
 constexpr bool half_tail(uint32_t groups) { return groups % kCG == kCG / 2 && groups > kCG; }
 
 // Q4 weights staged through LDS (coalesced 128-byte row loads by the whole
@@ -600,7 +602,7 @@ __device__ __forceinline__ void grouped_tile(const GroupedLaunch& p, const ProjP
   };
   // only a K that is not a multiple of the chunk has a tail chunk
   auto tail_chunk = [&](uint32_t c) { return TAIL && (c + 1) * kCG > G; };
-  // first group of chunk c (kTailHalf: the last chunk is the row's last eight
+  // first group of chunk c (HALF: the last chunk is the row's last eight
   // groups, of which the upper four are new)
   auto first_group = [&](uint32_t c) { return HALF ? min(c * kCG, G - kCG) : c * kCG; };
   // epilogue of slice s: lane holds rows 4*(lane/16) + i of every row block, column lane%16
@@ -1773,9 +1775,10 @@ hipError_t grouped_go(const char* family, const GroupedLaunch& p, uint32_t max_t
   }
   if (p.tile_rows != 0 && p.tile_rows != static_cast<uint32_t>(tile_rows<EPI>())) return hipErrorInvalidValue;
   if constexpr (EPI == kEpiRows) {
-    if (half && p.weights_once)
-      return grouped_go_k<EPI, WAVES, NBW, PROJ, false, true, true>(family, p, max_tiles, stream);
-    if (half) return grouped_go_k<EPI, WAVES, NBW, PROJ, false, false, true>(family, p, max_tiles, stream);
+    // half tails at the usual height are calls whose experts mostly hold one tile
+    // (above 48 rows per expert they take the tall tiles)
+    if (half && !p.weights_once) return hipErrorInvalidValue;
+    if (half) return grouped_go_k<EPI, WAVES, NBW, PROJ, false, true, true>(family, p, max_tiles, stream);
   }
   if (!whole) return grouped_go_k<EPI, WAVES, NBW, PROJ, true, false>(family, p, max_tiles, stream);
   if (lds_weights<EPI, false>() && p.weights_once)
