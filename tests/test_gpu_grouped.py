@@ -545,3 +545,23 @@ def test_down_gemm_of_whole_rows_at_half_chunks_over(device, hidden, inter):
         assert torch.equal(out.view(torch.int16), tall[:tokens].view(torch.int16)), tokens
     _, _, _, d_out, _ = mo.execute(x_np[:20], inds[:20], np_packs, "bf16", qmm=True)
     _close_qmm(host(tall[:20]), d_out, f"hidden {hidden}, inter {inter}")
+
+
+@pytest.mark.parametrize("hidden", [96, 1088])
+def test_down_gemm_of_half_chunks_gives_one_result_by_every_way(device, hidden):
+    """Inter 1152, whose half chunk over is too wide for k_down_rows: calls of few blocks let the lanes fetch their
+    own weights, larger ones stage them, calls above 48 rows per expert take 96-row tiles.  One row, the same bits."""
+    experts, k, inter, more = 96, 3, 1152, 1700
+    np_packs = packs(88, hidden, inter, experts)
+    rng = np.random.default_rng(89 + hidden)
+    inds = np.stack([rng.choice(experts, k, replace=False) for _ in range(more)]).astype(np.int32)
+    x_np = mo.bf16r(rng.normal(size=(more, hidden)).astype(np.float32))
+    switch = _switch(np_packs, hidden, inter, experts, device)
+    x, i = bf16_device(x_np, device), torch.tensor(inds, device=device)
+    tall = grouped_experts(switch, x, i)
+    for tokens in (20, 150, 1500):
+        out = grouped_experts(switch, x[:tokens].contiguous(), i[:tokens].contiguous())
+        torch.cuda.synchronize()
+        assert torch.equal(out.view(torch.int16), tall[:tokens].view(torch.int16)), tokens
+    _, _, _, d_out, _ = mo.execute(x_np[:20], inds[:20], np_packs, "bf16", qmm=True)
+    _close_qmm(host(tall[:20]), d_out, f"hidden {hidden}")

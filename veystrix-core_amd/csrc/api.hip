@@ -8,6 +8,7 @@
 
 #include <atomic>
 
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -1107,6 +1108,15 @@ struct GroupedExperts {
   bool counted;  // the sort's counters were zeroed by the router GEMM
 };
 
+// Down tiles of the usual height of a call whose pairs spread evenly over the
+// experts: one for every expert that some pair names, and for a growing share of
+// them a second once they average more than two thirds of a tile's rows.
+static uint32_t expected_down_tiles(uint32_t pairs, uint32_t experts) {
+  const double mean = double(pairs) / experts, most = vm::kGroupedRowsDown * 2 / 3;
+  const double second = mean > most ? (mean - most) / (vm::kGroupedRowsDown - most) : 0.0;
+  return static_cast<uint32_t>(experts * (second - std::expm1(-mean)) + 0.5);
+}
+
 static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char* ws, hipStream_t stream) {
   // the chunked GEMM addresses its activation matrices with 32-bit byte
   // offsets and its outputs with 32-bit element indices
@@ -1192,6 +1202,10 @@ static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char
   q.a_stride = g.I;
   q.a_rows = g.T * g.K + (g.shared ? g.T : 0);
   q.weights_once = uint64_t(g.T) * g.K <= uint64_t(g.E) * vm::kGroupedRowsDown;
+  if (!w.small && !whole_rows) {
+    q.live_tiles = expected_down_tiles(g.T * g.K, g.E) + (g.shared ? (g.T + vm::kGroupedRowsDown - 1) / vm::kGroupedRowsDown : 0);
+    q.cus = device_cus();
+  }
   q.tile_rows = w.small || w.tile_rows_dn == vm::kGroupedRowsDown ? 0u : w.tile_rows_dn;
   q.tiles = s.tiles_dn;
   q.tile_count = s.tile_count_dn;

@@ -1776,9 +1776,14 @@ hipError_t grouped_go(const char* family, const GroupedLaunch& p, uint32_t max_t
   if (p.tile_rows != 0 && p.tile_rows != static_cast<uint32_t>(tile_rows<EPI>())) return hipErrorInvalidValue;
   if constexpr (EPI == kEpiRows) {
     // half tails at the usual height are calls whose experts mostly hold one tile
-    // (above 48 rows per expert they take the tall tiles)
+    // (above 48 rows per expert they take the tall tiles).  Where every live
+    // block has a CU to itself, nothing hides the staged loads' latency and the
+    // lanes' own loads are the faster: hidden 1024 / inter 1152, four of 64
+    // experts, 500 rows (256 blocks) 72 us per call and 80 staged, 600 rows (267)
+    // 90 and 83
     if (half && !p.weights_once) return hipErrorInvalidValue;
-    if (half) return grouped_go_k<EPI, WAVES, NBW, PROJ, false, true, true>(family, p, max_tiles, stream);
+    if (half && p.live_tiles * ((p.n_dim + WAVES * NBW * 16 - 1) / (WAVES * NBW * 16)) > p.cus)
+      return grouped_go_k<EPI, WAVES, NBW, PROJ, false, true, true>(family, p, max_tiles, stream);
   }
   if (!whole) return grouped_go_k<EPI, WAVES, NBW, PROJ, true, false>(family, p, max_tiles, stream);
   if (lds_weights<EPI, false>() && p.weights_once)

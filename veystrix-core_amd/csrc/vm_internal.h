@@ -271,6 +271,7 @@ struct GroupedLaunch {
   uint32_t spb;                // column slices per block (set by launch_grouped)
   uint32_t tile_rows;          // rows per tile of `tiles`: 0 the instance's own, or kGroupedRowsTall (gate/up)
   bool weights_once;           // most groups hold one row tile: stream the weights past the L2
+  uint32_t live_tiles, cus;    // down GEMM: estimate of the tiles a call of evenly spread routes has, and the CUs
   // router GEMM only: block 0 zeroes zero_count words at zero_words (the
   // counters of the sort that follows the select)
   uint32_t* zero_words;
