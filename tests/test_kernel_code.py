@@ -10,7 +10,7 @@ import pytest
 
 from veymoe import build
 
-Kernel = namedtuple("Kernel", "vgprs scratch wave_barriers")
+Kernel = namedtuple("Kernel", "vgprs scratch sgpr_spills wave_barriers")
 _COMPILED = {}
 
 
@@ -32,8 +32,9 @@ def _kernels(source, tmp_path_factory):
             if m.group(1) not in meta:
                 continue
             value = lambda key: int(re.search(rf"\.amdhsa_{key} (\d+)", meta[m.group(1)]).group(1))
+            spills = re.search(rf"\.name: +{re.escape(m.group(1))}\n(?:    \..*\n)*?    \.sgpr_spill_count: (\d+)", text)
             found[m.group(1)] = Kernel(value("next_free_vgpr"), value("private_segment_fixed_size"),
-                                       m.group(0).count("; wave barrier"))
+                                       int(spills.group(1)), m.group(0).count("; wave barrier"))
         _COMPILED[source] = found
     return _COMPILED[source]
 
@@ -61,6 +62,15 @@ def test_decode_kernels_take_no_scratch(tmp_path_factory):
     kernels = _kernels("decode.hip", tmp_path_factory)
     for name, k in {**_instances(kernels, "k_gateupINS_"), **_instances(kernels, "k_downINS_")}.items():
         assert k.scratch == 0, (name, k)
+
+
+def test_float32_gateup_keeps_its_scalars(tmp_path_factory):
+    """The fp32 gate/up of several groups per lane, whose row index in a scalar had cost 180 spills to VGPR lanes."""
+    found = {name: k for name, k in _instances(_kernels("decode.hip", tmp_path_factory), "k_gateupINS_6ActF32E").items()
+             if "ELi64ELi2E" in name or "ELi64ELi4E" in name}
+    assert found
+    for name, k in found.items():
+        assert k.sgpr_spills <= 40, (name, k)
 
 
 def test_folded_down_runs_two_blocks_per_cu(tmp_path_factory):

@@ -59,7 +59,9 @@ constexpr int kGateupRowsPerLane = VM_GATEUP_ROWS;
 // waves per gate/up block: two for one token, whose few blocks are spread over
 // more CUs so; four for more tokens, where half as many blocks repeat the
 // selection (hidden 2048: 2 / 5 / 8 tokens 20.7 / 39.4 / 53.7 us per layer with
-// two, 20.0 / 38.5 / 52.8 with four; hidden 2560 the same within 1 %)
+// two, 20.0 / 38.5 / 52.8 with four; hidden 2560 the same within 1 %); fp32 rows
+// of several groups per lane keep two, their registers leave few waves per SIMD
+// (hidden 7168 / inter 2048, five tokens 735 us per layer with two, 788 with four)
 constexpr int kGuWaves = 2, kGuWavesMulti = 4;
 template <class A, bool GATE = false>
 __device__ void select_body(const SelectLaunch& p) {
@@ -200,7 +202,10 @@ __global__ __launch_bounds__(WAVES * 64) void k_gateup(GateUpLaunch p) {
 
   const uint32_t tid = threadIdx.x;
   const uint32_t lane = tid & 63u;
-  const uint32_t wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // a scalar, and with it the rows' base; in fp32 with several groups per lane
+  // that is one too many (180 SGPR spills at four groups: hidden 7168 / inter
+  // 2048, one / five tokens 154 / 735 us per layer, 148 / 702 per lane)
+  const uint32_t wave = A::kBytes == 4 && GI > 1 ? tid >> 6 : __builtin_amdgcn_readfirstlane(tid >> 6);
   typename Cand<A>::T* s_cand = s_cands[wave];
   const uint32_t lr = lane % LPR;
   const uint32_t rw = lane / LPR;
@@ -700,7 +705,9 @@ hipError_t gateup_launch(const GateUpLaunch& p, hipStream_t stream) {
 
 template <class A, int LPR, int GI, int U, int FOLD = 0>
 hipError_t gateup_go(const GateUpLaunch& p, hipStream_t stream) {
-  if (p.tokens > 1) return gateup_launch<A, LPR, GI, U, FOLD, kGuWavesMulti>(p, stream);
+  if constexpr (A::kBytes == 2 || GI == 1) {
+    if (p.tokens > 1) return gateup_launch<A, LPR, GI, U, FOLD, kGuWavesMulti>(p, stream);
+  }
   return gateup_launch<A, LPR, GI, U, FOLD, kGuWaves>(p, stream);
 }
 
