@@ -524,11 +524,11 @@ def test_small_calls_of_one_supported_size_give_the_larger_calls_bits(device, hi
     assert torch.equal(small.view(torch.int16), large[:40].view(torch.int16))
 
 
-@pytest.mark.parametrize("inter", [384, 640, 896])
+@pytest.mark.parametrize("inter", [256, 384, 640, 896])
 @pytest.mark.parametrize("hidden", [1088, 2080])
 def test_down_gemm_of_whole_rows_at_half_chunks_over(device, hidden, inter):
     """Every instance of k_down_rows whose K has half a chunk over, with two column blocks per wave (hidden 1088) and
-    four (2080), both ending inside a block: the bits of the chunked GEMM's 96-row tiles, which a call of 500 tokens
+    four (2080), both ending inside a block, and K of one chunk, which is the chunked GEMM's at hidden 2080: the bits of the chunked GEMM's 96-row tiles, which a call of 500 tokens
     takes, and the oracle's values.  Calls of 20 and 150 tokens; two thirds of the rows go to the last expert."""
     experts, k, more = 24, 3, 500
     np_packs = packs(86, hidden, inter, experts)

@@ -1142,7 +1142,7 @@ static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char
   s.shared_rows = g.shared ? g.T : 0;
   s.tile_rows = w.tile_rows;
   s.tile_rows_dn = w.tile_rows_dn;
-  const bool whole_rows = !w.small && w.tile_rows_dn == vm::kGroupedRowsDown && vm::down_rows_supported(g.I);
+  const bool whole_rows = !w.small && w.tile_rows_dn == vm::kGroupedRowsDown && vm::down_rows_supported(g.I, g.H);
   // one output row per token and slot: k_down_rows stores there itself instead
   // of leaving the sorted rows for a copy (700 rows of hidden 1024, 64 experts
   // top-4: 34.8 -> 30.8 us per call)

@@ -1893,18 +1893,18 @@ hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipS
   return hipErrorInvalidValue;
 }
 
-// k_down_rows takes K of one chunk, and of half a chunk over whole ones up to
-// 896 (102 KB of LDS there, one block per CU).  Where the chunked GEMM runs
-// whole chunks, two and more, it is the better one: per call, ten of 512
-// experts, 1000 rows, hidden 2048 / inter 512 291 us chunked and 305 so, 2560 /
-// 768 531 and 549, but 2560 / 384 334 and 315, 2560 / 896 669 and 645.  Calls of
-// few blocks gain too (hidden 1024, four of 64 experts, 24 rows: inter 384 39.4
-// and 35.0, inter 896 55.3 and 48.4).
+// k_down_rows takes K of half a chunk over whole ones up to 896 (102 KB of LDS
+// there, one block per CU), and of one chunk below hidden 2048.  Where the
+// chunked GEMM runs whole chunks and fills the chip, it is the better one: per
+// call, ten of 512 experts, 1000 rows, hidden 2048 / inter 512 291 us chunked
+// and 305 so, 2560 / 768 531 and 549, 2560 / 256 207 and 222, but 2560 / 384 334
+// and 315, 2560 / 896 669 and 645.  Calls of few blocks gain (hidden 1024, four
+// of 64 experts, 24 rows: inter 384 39.4 and 35.0, inter 896 55.3 and 48.4; inter
+// 256, 333 rows 41.8 and 38.8).
 constexpr uint32_t kDownRowsGroups = 28;
 // Column blocks per wave (SPB): four from hidden 2048 up (2560 / 640, 1999 rows:
 // 551 us per call with two, 539 with four), two below, where four leave the chip
-// idle (1024 / 640, four of 64 experts, 400 rows: 57.3 with four, 51.4 with two)
-// and at K = 256.
+// idle (1024 / 640, four of 64 experts, 400 rows: 57.3 with four, 51.4 with two).
 constexpr uint32_t kDownRowsWide = 2048;
 
 template <int QG, int SPB, bool SLOTS>
@@ -1932,9 +1932,9 @@ hipError_t down_rows_go_k(const GroupedLaunch& p, uint32_t max_tiles, hipStream_
   return hipGetLastError();
 }
 
-bool down_rows_supported(uint32_t k_dim) {
+bool down_rows_supported(uint32_t k_dim, uint32_t n_dim) {
   const uint32_t groups = k_dim / kGroup;
-  return groups == kCG || (half_tail(groups) && groups <= kDownRowsGroups);
+  return groups == kCG ? n_dim < kDownRowsWide : half_tail(groups) && groups <= kDownRowsGroups;
 }
 
 template <int QG>
@@ -1948,7 +1948,7 @@ hipError_t down_rows_go(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t 
 }
 
 hipError_t launch_down_rows(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream) {
-  if (p.a_stride != p.k_dim || p.row_token != nullptr || !down_rows_supported(p.k_dim)) return hipErrorInvalidValue;
+  if (p.a_stride != p.k_dim || p.row_token != nullptr || !down_rows_supported(p.k_dim, p.n_dim)) return hipErrorInvalidValue;
   switch (p.k_dim / kGroup) {
     case 8: return down_rows_go<2>(p, max_tiles, stream);
     case 12: return down_rows_go<3>(p, max_tiles, stream);

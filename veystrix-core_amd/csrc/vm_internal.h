@@ -335,7 +335,7 @@ bool rows_supported(uint32_t k_dim);
 hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream);
 // The down GEMM over tiles of up to kGroupedRowsDown rows with whole A rows in
 // LDS (k_down_rows).
-bool down_rows_supported(uint32_t k_dim);
+bool down_rows_supported(uint32_t k_dim, uint32_t n_dim);
 hipError_t launch_down_rows(const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream);
 // Calls up to this many (token, slot) pairs sort in one block.
 constexpr uint32_t kSortOneBlockPairs = 4096;
