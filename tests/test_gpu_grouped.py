@@ -528,8 +528,9 @@ def test_small_calls_of_one_supported_size_give_the_larger_calls_bits(device, hi
 @pytest.mark.parametrize("hidden", [1088, 2080])
 def test_down_gemm_of_whole_rows_at_half_chunks_over(device, hidden, inter):
     """Every instance of k_down_rows whose K has half a chunk over, with two column blocks per wave (hidden 1088) and
-    four (2080), both ending inside a block, and K of one chunk, which is the chunked GEMM's at hidden 2080: the bits of the chunked GEMM's 96-row tiles, which a call of 500 tokens
-    takes, and the oracle's values.  Calls of 20 and 150 tokens; two thirds of the rows go to the last expert."""
+    four (2080), both ending inside a block, and K of one chunk, which is the chunked GEMM's at hidden 2080: the bits
+    of the chunked GEMM's 96-row tiles, which a call of 500 tokens takes, and the oracle's values.  Calls of 20 and
+    150 tokens; two thirds of their rows go to the last expert."""
     experts, k, more = 24, 3, 500
     np_packs = packs(86, hidden, inter, experts)
     rng = np.random.default_rng(87 + inter + hidden)
@@ -565,3 +566,20 @@ def test_down_gemm_of_half_chunks_gives_one_result_by_every_way(device, hidden):
         assert torch.equal(out.view(torch.int16), tall[:tokens].view(torch.int16)), tokens
     _, _, _, d_out, _ = mo.execute(x_np[:20], inds[:20], np_packs, "bf16", qmm=True)
     _close_qmm(host(tall[:20]), d_out, f"hidden {hidden}")
+
+
+@pytest.mark.parametrize("hidden,inter,tokens", [(256, 640, 12), (256, 640, 150), (256, 256, 150), (256, 1152, 150),
+                                                 (256, 640, 300), (2048, 640, 300), (2048, 640, 400)])
+def test_grouped_layer_with_a_shared_expert_over_half_chunks(device, hidden, inter, tokens):
+    """The shared expert's rows as one more group of the whole-row and the chunked down GEMM (up to 256 rows), and on
+    the side stream in tiles of the usual height (300 rows: few blocks) and in tall ones (400 rows at hidden 2048)."""
+    spec = synth.LayerSpec("half_shared", hidden, inter, 24, 4, inter, 1)
+    seed = 340 + inter + tokens
+    layer = assemble.build_layer(spec, seed, device, dense=True)
+    x_np = mo.bf16_bits_to_f32(synth.tokens(spec, seed, tokens))
+    y = layer(bf16_device(x_np, device))
+    torch.cuda.synchronize()
+    rows = np.unique(np.linspace(0, tokens - 1, 40).astype(int))
+    ref = _layer_ref(spec, seed, x_np, rows)
+    same = _check_selection(layer.last_inds.cpu().numpy()[rows], ref, spec.top_k, 3, f"T={tokens}")
+    _assert_layer(host(y)[rows], spec, seed, x_np, rows, same, ref, f"{hidden}/{inter} T={tokens}")

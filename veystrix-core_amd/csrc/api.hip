@@ -1108,6 +1108,8 @@ struct GroupedExperts {
   bool counted;  // the sort's counters were zeroed by the router GEMM
 };
 
+static uint32_t usual_down_tiles(uint32_t rows) { return (rows + vm::kGroupedRowsDown - 1) / vm::kGroupedRowsDown; }
+
 // Down tiles of the usual height of a call whose pairs spread evenly over the
 // experts: one for every expert that some pair names, and for a growing share of
 // them a second once they average more than two thirds of a tile's rows.
@@ -1202,10 +1204,9 @@ static int run_grouped_experts(const GroupedExperts& g, const GroupedWs& w, char
   q.a_stride = g.I;
   q.a_rows = g.T * g.K + (g.shared ? g.T : 0);
   q.weights_once = uint64_t(g.T) * g.K <= uint64_t(g.E) * vm::kGroupedRowsDown;
-  if (!w.small && !whole_rows) {
-    q.live_tiles = expected_down_tiles(g.T * g.K, g.E) + (g.shared ? (g.T + vm::kGroupedRowsDown - 1) / vm::kGroupedRowsDown : 0);
-    q.cus = device_cus();
-  }
+  if (!w.small && !whole_rows && vm::down_half_tail(g.I))
+    q.few_blocks = (expected_down_tiles(g.T * g.K, g.E) + (g.shared ? usual_down_tiles(g.T) : 0u)) *
+                       vm::down_slices(g.H) <= device_cus();
   q.tile_rows = w.small || w.tile_rows_dn == vm::kGroupedRowsDown ? 0u : w.tile_rows_dn;
   q.tiles = s.tiles_dn;
   q.tile_count = s.tile_count_dn;
@@ -1273,8 +1274,13 @@ static hipError_t launch_shared_expert(const VmLayerArgs* a, uint16_t* sig, uint
   q.a = sh_act;
   // its own group of T rows: tall tiles above 48 rows (each
   // weight dequantised half as often, which leaves the routed gate/up it runs
-  // beside more of the CUs)
-  const uint32_t trd = down_tile_rows(T, 1, I, 1);
+  // beside more of the CUs).  With half a chunk over and so few blocks that they
+  // are a chain of latencies, a quarter of the CUs, tiles of the usual height
+  // whose lanes fetch their own weights (hidden 1024 / inter 1152, four of 64
+  // experts, 333 rows, 28 blocks: 84 us per call, 92 with tall tiles; 2048 / 640,
+  // eight of 128, 700 rows, 120 blocks: 159 and 153)
+  q.few_blocks = vm::down_half_tail(I) && usual_down_tiles(T) * vm::down_slices(H) * 4 <= device_cus();
+  const uint32_t trd = q.few_blocks ? vm::kGroupedRowsDown : down_tile_rows(T, 1, I, 1);
   q.tile_rows = trd == vm::kGroupedRowsDown ? 0u : trd;
   q.shared[0] = to_ptrs(a->shared_down_proj);
   q.shared[1] = vm::ProjPtrs{};

@@ -1777,13 +1777,13 @@ hipError_t grouped_go(const char* family, const GroupedLaunch& p, uint32_t max_t
   if constexpr (EPI == kEpiRows) {
     // half tails at the usual height are calls whose experts mostly hold one tile
     // (above 48 rows per expert they take the tall tiles).  Where every live
-    // block has a CU to itself, nothing hides the staged loads' latency and the
-    // lanes' own loads are the faster: hidden 1024 / inter 1152, four of 64
-    // experts, 500 rows (256 blocks) 72 us per call and 80 staged, 600 rows (267)
-    // 90 and 83
-    if (half && !p.weights_once) return hipErrorInvalidValue;
-    if (half && p.live_tiles * ((p.n_dim + WAVES * NBW * 16 - 1) / (WAVES * NBW * 16)) > p.cus)
-      return grouped_go_k<EPI, WAVES, NBW, PROJ, false, true, true>(family, p, max_tiles, stream);
+    // block has a CU to itself (few_blocks), nothing hides the staged loads'
+    // latency and the lanes' own loads are the faster: hidden 1024 / inter 1152,
+    // four of 64 experts, 500 rows (256 blocks) 72 us per call and 80 staged, 600
+    // rows (267) 90 and 83
+    if (half && !p.few_blocks)
+      return p.weights_once ? grouped_go_k<EPI, WAVES, NBW, PROJ, false, true, true>(family, p, max_tiles, stream)
+                            : hipErrorInvalidValue;
   }
   if (!whole) return grouped_go_k<EPI, WAVES, NBW, PROJ, true, false>(family, p, max_tiles, stream);
   if (lds_weights<EPI, false>() && p.weights_once)
@@ -1836,9 +1836,11 @@ hipError_t launch_grouped(int epi, const GroupedLaunch& p, uint32_t max_tiles, h
 // LDS).  Other K take the chunked GEMM.
 constexpr uint32_t kRowsMaxK = 4096;
 
-bool down_tall_supported(uint32_t k_dim) {
-  return (k_dim / kGroup) % kCG == 0 || half_tail(k_dim / kGroup);
-}
+bool down_half_tail(uint32_t k_dim) { return half_tail(k_dim / kGroup); }
+
+bool down_tall_supported(uint32_t k_dim) { return (k_dim / kGroup) % kCG == 0 || down_half_tail(k_dim); }
+
+uint32_t down_slices(uint32_t n_dim) { return (n_dim + VM_DN_WAVES * VM_DN_NBW * 16 - 1) / (VM_DN_WAVES * VM_DN_NBW * 16); }
 
 bool rows_supported(uint32_t k_dim) {
   return k_dim == 256 || k_dim == 512 || k_dim == 1024 || k_dim == 2048 || k_dim == kRowsMaxK;

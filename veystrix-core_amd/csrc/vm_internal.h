@@ -271,7 +271,7 @@ struct GroupedLaunch {
   uint32_t spb;                // column slices per block (set by launch_grouped)
   uint32_t tile_rows;          // rows per tile of `tiles`: 0 the instance's own, or kGroupedRowsTall (gate/up)
   bool weights_once;           // most groups hold one row tile: stream the weights past the L2
-  uint32_t live_tiles, cus;    // down GEMM: estimate of the tiles a call of evenly spread routes has, and the CUs
+  bool few_blocks;             // down GEMM, half a chunk over: the lanes fetch their own weights (see grouped_go)
   // router GEMM only: block 0 zeroes zero_count words at zero_words (the
   // counters of the sort that follows the select)
   uint32_t* zero_words;
@@ -331,6 +331,9 @@ hipError_t launch_grouped(int epi, const GroupedLaunch& p, uint32_t max_tiles, h
 constexpr int kRowsTile = 16;
 // The down GEMM's staged-weight instances (and so its tall tiles) take this K.
 bool down_tall_supported(uint32_t k_dim);
+// K of half a chunk over, and the column slices of the chunked down GEMM.
+bool down_half_tail(uint32_t k_dim);
+uint32_t down_slices(uint32_t n_dim);
 bool rows_supported(uint32_t k_dim);
 hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream);
 // The down GEMM over tiles of up to kGroupedRowsDown rows with whole A rows in
