@@ -89,6 +89,10 @@ def test_hyper_mix_tiles_match_the_oracle_and_the_per_token_kernels(device, hc, 
     base = normed_bytes + (2 * T * r + 255) // 256 * 256
     ws = hyper._ws[(T, 0, xd.device)]
     assert ws.numel() > base
+    ws[base:] = 0xcd
+    mixed, _, weights = hyper(xd)
+    torch.cuda.synchronize()
+    assert bool((ws[base:] != 0xcd).any()), "the tile kernels wrote nothing"
     normed = ws[: 2 * T * n].clone()
     low = ws[normed_bytes: normed_bytes + 2 * T * r].clone().view(torch.bfloat16)
     hyper._ws[(T, 0, xd.device)] = torch.zeros(base, dtype=torch.uint8, device=device)
@@ -102,6 +106,85 @@ def test_hyper_mix_tiles_match_the_oracle_and_the_per_token_kernels(device, hc, 
     want_m, want_w, _ = go.hyper_mix(x, *parts, hc, 1e-6, group_size=group, one_centered=one_centered)
     assert_close(host(weights), want_w, f"weights T={T}")
     assert_close(host(mixed), want_m, f"mixed T={T}")
+
+
+def _tiles_and_per_token(hyper, xd, r):
+    """(mixed, weights) of a call on 16-token tiles, whose scratch behind the workspace's base it must have written,
+    and of the same call from a workspace without that scratch, which runs the per-token kernels."""
+    T, n = xd.shape
+    hyper(xd)
+    key = (T, 0, xd.device)
+    base = (2 * T * n + 255) // 256 * 256 + (2 * T * r + 255) // 256 * 256
+    ws = hyper._ws[key]
+    ws[base:] = 0xcd
+    mixed, _, weights = hyper(xd)
+    torch.cuda.synchronize()
+    assert bool((ws[base:] != 0xcd).any()), "the tile kernels wrote nothing"
+    hyper._ws[key] = torch.zeros(base, dtype=torch.uint8, device=xd.device)
+    mixed1, _, weights1 = hyper(xd)
+    torch.cuda.synchronize()
+    hyper._ws[key] = ws
+    return (mixed.clone(), weights.clone()), (mixed1, weights1)
+
+
+def _power_of_two_inject(exps, hc, n, device):
+    """Injection projection of ones: row j scales the 128 columns of block b by 2 ** exps[b * hc + j]."""
+    scales = np.ldexp(np.float32(1), np.asarray(exps).reshape(n // 128, hc)).astype(np.float32)
+    scales = np.repeat(scales.T, 4, axis=1)                                  # four groups of 32 per block
+    words = np.full((hc, n // 8), 0x11111111, np.uint32)
+    return assemble.projection(words, mo.f32_to_bf16_bits(scales), np.zeros((hc, n // 32), np.uint16), device)
+
+
+@pytest.mark.parametrize("hc,exps", [(8, range(-130, 126)), (1, [*range(-133, -128), 126, 127] + [127] * 25)],
+                         ids=["-133..122", "ends"])
+def test_hyper_weights_pin_the_sigmoid_over_the_bf16_values(device, hc, exps):
+    """The injection weights are 2 * sigmoid(a): with one value of every token's row set, a runs over the bf16 values
+    of both signs, all 128 significands of each power of two from the smallest subnormal to the largest finite one, and
+    over infinity and NaN; bit for bit the oracle's op-by-op sigmoid, from the tile and from the per-token kernels."""
+    n, r = 4096, 32
+    H = n // hc
+    col = np.arange(n)
+    gain = ((128 + col % 128) / 128.0 / 64.0).astype(np.float32)             # normalised, 64 * gain: 1 .. 255/128
+    zero = lambda rows, width: assemble.projection(np.zeros((rows, width // 8), np.uint32),
+                                                   np.zeros((rows, width // 32), np.uint16),
+                                                   np.zeros((rows, width // 32), np.uint16), device)
+    hyper = HyperConnection(torch.from_numpy(gain).to(device).to(torch.bfloat16), zero(r, n), zero(n, r),
+                            _power_of_two_inject(exps, hc, n, device), hc, eps=1e-30)
+    x = torch.zeros((2 * n + 1, n), dtype=torch.bfloat16, device=device)
+    x[torch.arange(n), torch.arange(n)] = 1.0
+    x[n + torch.arange(n), torch.arange(n)] = -1.0
+    x[2 * n, 0] = float("nan")
+    (_, tiles), (_, per_token) = _tiles_and_per_token(hyper, x, r)
+    power = np.asarray(exps).reshape(n // 128, hc)[col // 128]               # [n, hc]
+    with np.errstate(over="ignore", under="ignore"):
+        a = np.ldexp((128 + col % 128)[:, None] / 128.0, power).astype(np.float32)
+        a = mo.bf16r(mo.bf16r(a) / np.float32(hc))
+    a = np.concatenate([a, -a])
+    with np.errstate(over="ignore"):
+        want = mo.f32_to_bf16_bits(mo.bf16r(np.float32(2) * mo.sigmoid(a, "bf16")))
+    for got, what in ((tiles, "tiles"), (per_token, "per token")):
+        bits = got.view(torch.int16).cpu().numpy().view(np.uint16)
+        np.testing.assert_array_equal(bits[:-1], want, err_msg=what)
+        assert bool(torch.isnan(got[-1].float()).all()), what
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), -float("inf")])
+def test_hyper_mix_tiles_keep_a_bad_token_to_itself(device, bad):
+    """One stream value that is not finite: its token's outputs are what the per-token kernels make of it (NaN), every
+    other token's, in the same tile too, the bits of the call without it."""
+    hc, H, r, T = 4, 2560, 32, 67
+    rng = np.random.default_rng(SEED + 11)
+    hyper = _hyper_dev(_hyper_np(rng, hc, H, r), hc, device)
+    _, xd = _streams(rng, T, hc * H, device)
+    (clean_m, clean_w), _ = _tiles_and_per_token(hyper, xd, r)
+    xd[35, 4321] = bad
+    (mixed, weights), (mixed1, weights1) = _tiles_and_per_token(hyper, xd, r)
+    rest = [t for t in range(T) if t != 35]
+    assert torch.equal(mixed[rest].view(torch.int16), clean_m[rest].view(torch.int16))
+    assert torch.equal(weights[rest].view(torch.int16), clean_w[rest].view(torch.int16))
+    for got, one in ((mixed[35], mixed1[35]), (weights[35], weights1[35])):
+        assert bool(torch.isnan(got.float()).any())
+        assert torch.equal(torch.isnan(got.float()), torch.isnan(one.float()))
 
 
 def test_hyper_mix_float32(device):
@@ -167,6 +250,34 @@ def test_injection_in_the_experts_epilogue_is_exact(device, T, in_place):
     torch.cuda.synchronize()
     assert torch.equal(y2.view(torch.int16), y.view(torch.int16))
     np.testing.assert_array_equal(host(target), want)
+
+
+@pytest.mark.parametrize("hidden,inter", [(256, 640), (1280, 320), (256, 1280)])
+@pytest.mark.parametrize("T,dtype", [(1, torch.bfloat16), (5, torch.bfloat16), (3, torch.float32)])
+def test_injection_over_folded_down_rows_is_exact(device, hidden, inter, T, dtype):
+    """The injecting down instances of rows a quarter over a power of two (10, 20 and 40 groups): the plain call's
+    output, and its injection, in bf16 to the bit."""
+    hc = 3
+    spec = synth.LayerSpec("glue_folded", hidden, inter, 16, 4, inter, 1)
+    layer = assemble.build_layer(spec, SEED, device, dense=True)
+    rng = np.random.default_rng(SEED + inter + T)
+    x = assemble.tokens_tensor(spec, SEED, device, T, stream=9).to(dtype)
+    streams = torch.from_numpy(mo.bf16r(rng.normal(0, 1, (T, hc * hidden)).astype(np.float32))).to(device).to(dtype)
+    weights = torch.from_numpy(mo.bf16r(rng.uniform(0, 2, (T, hc)).astype(np.float32))).to(device).to(dtype)
+    plain = layer.forward(x).clone()
+    target = torch.empty_like(streams)
+    y = layer.forward(x, inject=(streams, weights, target))
+    torch.cuda.synchronize()
+    assert torch.equal(y, plain)
+    if dtype == torch.bfloat16:
+        np.testing.assert_array_equal(host(target), go.inject(host(streams), host(y), host(weights)))
+    else:
+        # the product may be fused into the sum: its own rounding is then missing, half a step of the product, which
+        # can move the sum's rounding by one more half step
+        product = y.unsqueeze(1) * weights.unsqueeze(2)
+        want = streams.view(T, hc, hidden) + product
+        bound = 2.0 ** -24 * product.abs() + 2.0 ** -23 * want.abs()
+        assert bool(((target.view(T, hc, hidden) - want).abs() <= bound).all())
 
 
 def test_mlp_branch_matches_the_oracle_chain(device):

@@ -22,7 +22,8 @@ import torch
 
 from gpu_util import bf16_device, host, packs, to_device, ulp_diff_bf16
 from oracle import moe_oracle as mo
-from veymoe import assemble, synth
+from veymoe import _lib, assemble, synth
+from veymoe.device import ptr, stream_handle
 from veymoe.grouped import COMBINE_FUSED, COMBINE_GENERIC, COMBINE_NONE, grouped_experts
 from veymoe.layer import HipSwitchGLU
 from veymoe.layout import RecordLayout, pack_record
@@ -583,3 +584,54 @@ def test_grouped_layer_with_a_shared_expert_over_half_chunks(device, hidden, int
     ref = _layer_ref(spec, seed, x_np, rows)
     same = _check_selection(layer.last_inds.cpu().numpy()[rows], ref, spec.top_k, 3, f"T={tokens}")
     _assert_layer(host(y)[rows], spec, seed, x_np, rows, same, ref, f"{hidden}/{inter} T={tokens}")
+
+
+@pytest.mark.parametrize("inter", [256, 640])
+@pytest.mark.parametrize("tokens", [30, 150])
+def test_down_gemm_of_whole_rows_over_pool_records(device, inter, tokens):
+    """k_down_rows over records behind a slot table, one record a load past whose end would leave the pool: the dense
+    bits; experts without a record set the status bit and leave rows of zeros, in the slot rows and in the combine."""
+    hidden, experts, k = 1088, 24, 3
+    np_packs = packs(90, hidden, inter, experts)
+    rng = np.random.default_rng(91 + inter)
+    inds_np = np.stack([rng.choice(experts, k, replace=False) for _ in range(tokens)]).astype(np.int32)
+    inds = torch.tensor(inds_np, device=device)
+    x = bf16_device(mo.bf16r(rng.normal(size=(tokens, hidden)).astype(np.float32)), device)
+    scores = torch.rand((tokens, k), device=device).to(torch.bfloat16)
+    dense = _switch(np_packs, hidden, inter, experts, device)
+    layout = RecordLayout(hidden, inter)
+    pool = ExpertPool(layout, experts, layers=1, experts=experts, device=device)
+    slots = rng.permutation(experts)
+    for e in range(experts):
+        parts = {(name, part): np_packs[name][i][e] for name in np_packs
+                 for i, part in enumerate(("weight", "scales", "biases"))}
+        pool.record(int(slots[e])).copy_(torch.from_numpy(pack_record(parts, layout)))
+    pool.place_all(0, slots)
+    pooled = HipSwitchGLU(hidden, inter, experts, pool=pool, layer_id=0)
+    rows = grouped_experts(dense, x, inds)
+    assert torch.equal(grouped_experts(pooled, x, inds), rows)
+
+    hole = int(inds_np[0, 0])
+    table = pool.table(0).clone()
+    table[hole] = -1
+    lib = _lib.lib()
+    for mode in (COMBINE_NONE, COMBINE_FUSED):
+        want = torch.where((inds == hole).unsqueeze(-1), torch.zeros_like(rows), rows)
+        if mode == COMBINE_FUSED:   # an expert of all-zero rows adds nothing to a token's sum
+            kept = torch.where(inds == hole, torch.full_like(inds, -1), inds)
+            want = grouped_experts(dense, x, kept, scores, None, mode)
+        out = torch.full_like(want, float("nan"))
+        status = torch.zeros(1, dtype=torch.int32, device=device)
+        ws = torch.empty(int(lib.vm_moe_grouped_workspace(tokens, k, hidden, inter, experts, 0)), dtype=torch.uint8,
+                         device=device)
+        a = _lib.VmGroupedArgs()
+        a.x, a.inds, a.output, a.status = ptr(x), ptr(inds), ptr(out), ptr(status)
+        a.scores = ptr(scores)
+        a.pool, a.slot_table = pool.view(), ptr(table)
+        a.workspace, a.workspace_bytes = ptr(ws), ws.numel()
+        a.tokens, a.top_k, a.hidden_size, a.inter_size, a.expert_count = tokens, k, hidden, inter, experts
+        a.group_size, a.act_dtype, a.combine_mode = 32, 0, mode
+        _lib.check(lib.vm_moe_grouped(a, stream_handle()))
+        torch.cuda.synchronize()
+        assert int(status.item()) & 1
+        assert torch.equal(out, want), mode

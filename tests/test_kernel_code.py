@@ -11,31 +11,42 @@ import pytest
 from veymoe import build
 
 Kernel = namedtuple("Kernel", "vgprs scratch sgpr_spills wave_barriers")
+SOURCES = ("grouped.hip", "decode.hip", "glue.hip")
 _COMPILED = {}
 
 
+def _listing(proc, listing):
+    """Kernel by mangled name of one finished compile."""
+    _, err = proc.communicate()
+    assert proc.returncode == 0, err[-2000:]
+    text = listing.read_text()
+    meta = {m.group(1): m.group(0) for m in re.finditer(r"\.amdhsa_kernel (\S+)\n.*?\.end_amdhsa_kernel", text, re.S)}
+    spills = dict(re.findall(r"\.name: +(\S+)\n(?:    \..*\n)*?    \.sgpr_spill_count: (\d+)", text))
+    found = {}
+    for m in re.finditer(r"^(_Z\S+):.*?^\.Lfunc_end\d+:", text, re.M | re.S):
+        name = m.group(1)
+        if name not in meta:
+            continue
+        value = lambda key: int(re.search(rf"\.amdhsa_{key} (\d+)", meta[name]).group(1))
+        found[name] = Kernel(value("next_free_vgpr"), value("private_segment_fixed_size"), int(spills[name]),
+                             m.group(0).count("; wave barrier"))
+    return found
+
+
 def _kernels(source, tmp_path_factory):
-    """Kernel by mangled name for one file of csrc, compiled once."""
-    if source not in _COMPILED:
+    """Kernel by mangled name for one file of csrc; the files are compiled once, side by side."""
+    if not _COMPILED:
         try:
             hipcc = build.hipcc()
         except RuntimeError:
             pytest.skip("hipcc is not installed")
-        listing = tmp_path_factory.mktemp("listing") / "device.s"
-        cmd = [hipcc, *build.HIP_FLAGS, "--cuda-device-only", "-S", os.path.join(build.CSRC, source), "-o", str(listing)]
-        proc = subprocess.run(cmd, capture_output=True, text=True)
-        assert proc.returncode == 0, proc.stderr[-2000:]
-        text = listing.read_text()
-        meta = {m.group(1): m.group(0) for m in re.finditer(r"\.amdhsa_kernel (\S+)\n.*?\.end_amdhsa_kernel", text, re.S)}
-        found = {}
-        for m in re.finditer(r"^(_Z\S+):.*?^\.Lfunc_end\d+:", text, re.M | re.S):
-            if m.group(1) not in meta:
-                continue
-            value = lambda key: int(re.search(rf"\.amdhsa_{key} (\d+)", meta[m.group(1)]).group(1))
-            spills = re.search(rf"\.name: +{re.escape(m.group(1))}\n(?:    \..*\n)*?    \.sgpr_spill_count: (\d+)", text)
-            found[m.group(1)] = Kernel(value("next_free_vgpr"), value("private_segment_fixed_size"),
-                                       int(spills.group(1)), m.group(0).count("; wave barrier"))
-        _COMPILED[source] = found
+        path = tmp_path_factory.mktemp("listings")
+        jobs = {}
+        for name in SOURCES:
+            out = path / f"{name}.s"
+            cmd = [hipcc, *build.HIP_FLAGS, "--cuda-device-only", "-S", os.path.join(build.CSRC, name), "-o", str(out)]
+            jobs[name] = subprocess.Popen(cmd, stdout=subprocess.DEVNULL, stderr=subprocess.PIPE, text=True), out
+        _COMPILED.update({name: _listing(*job) for name, job in jobs.items()})
     return _COMPILED[source]
 
 
@@ -79,3 +90,12 @@ def test_folded_down_runs_two_blocks_per_cu(tmp_path_factory):
     for name, k in _instances(_kernels("decode.hip", tmp_path_factory), "k_downINS_7ActBF16E").items():
         if "ELb0ELi4ELi4E" in name:  # no injection, folded, four row groups
             assert k.vgprs <= 80, (name, k)
+
+
+def test_hyper_connection_tiles_register_budgets(tmp_path_factory):
+    """k_hc_low runs three blocks of four waves per CU (at most 168 registers), k_hc_mix four for up to four streams
+    (128), else three; none spills."""
+    kernels = _kernels("glue.hip", tmp_path_factory)
+    for name, k in {**_instances(kernels, "k_hc_lowE"), **_instances(kernels, "k_hc_mixILb")}.items():
+        limit = 128 if "k_hc_mixILb1ELi4E" in name else 168
+        assert k.vgprs <= limit and k.scratch == 0, (name, k)
