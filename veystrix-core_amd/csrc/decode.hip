@@ -11,7 +11,7 @@
 //             slot's rank from the lanes' sorted keys by wave maxima
 //             (vm_select.h), maps the expert to its slot through the slot
 //             table entries it loaded beside the logits, and hands the route
-//             word to the block's other wave through LDS.  Every lane then
+//             word to the block's other waves through LDS.  Every lane then
 //             streams gate and up Q4/G32 rows against its activation groups
 //             held in registers; SwiGLU runs on the lanes that hold the row
 //             sums.  Shared-expert pairs skip the selection.  One block per
@@ -196,8 +196,8 @@ __global__ __launch_bounds__(WAVES * 64) void k_gateup(GateUpLaunch p) {
   constexpr int NF = FOLD ? (U + FOLD - 1) / FOLD : 0;  // folded loads per lane and projection
   constexpr int REM = FOLD ? LPR / FOLD : 1;            // groups over of a row
   static_assert(FOLD == 0 || GI == 1, "folded rows have one whole group per lane");
-  // every wave runs the selection itself (its own candidate list), so no
-  // barrier stands between the selection and the weight loads
+  // candidates of the selection: wave 0's list is used (one list for the block
+  // takes the folded instances back to a scratch frame)
   __shared__ typename Cand<A>::T s_cands[WAVES][kMaxCand];
 
   const uint32_t tid = threadIdx.x;
@@ -438,7 +438,11 @@ __global__ __launch_bounds__(kDownBlock, FOLD && !INJ && A::kBytes == 2 ? 6 : 3)
   // the CU (12 waves at 86 VGPRs), so the wave keeps its slot's activations in
   // LDS (16 bytes of padding per group: the lanes' reads are conflict-free) and
   // takes one group at a time: 80 VGPRs; hidden 2560 / inter 640, one / five /
-  // eight tokens 20.9 / 57.5 / 76.9 -> 20.3 / 52.1 / 70.0 us per layer.
+  // eight tokens 20.9 / 57.5 / 76.9 -> 20.3 / 52.1 / 70.0 us per layer.  The
+  // injecting and the fp32 instances (97-114) stay at one block; unfolded and
+  // with the longer unpacking an injecting layer took 25.0 / 78.3 / 115.6 us (two
+  // blocks), now 19.5 / 56.0 / 74.7, an fp32 one 31.3 / 94.3 / 139.5 and 22.9 /
+  // 71.6 / 96.0.
   constexpr int kUPG = kGroup * A::kBytes / 16;             // 16-byte units per group
   constexpr int kActG = FOLD ? LPR + LPR / (FOLD + !FOLD) : 1;  // groups of a row
   constexpr int kActU = (kActG * kUPG + 63) / 64;           // units per lane

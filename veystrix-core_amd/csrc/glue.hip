@@ -267,8 +267,8 @@ __global__ __launch_bounds__(kHcThreads) void k_hc_up(HcLaunch p) {
 //             stream, W_up rows as MFMA A rows in the order that leaves a lane
 //             eight consecutive outputs of one token.
 //
-// n = 10240, 700 tokens: 112 us per call before, 37.7 now (back to back in a
-// graph; 4096 tokens 595 and 119).  What is left is latency and VALU: about 30
+// n = 10240, 700 tokens: 112 us per call per token, 35.7 in tiles (back to back;
+// 4096 tokens 595 and 119).  What is left is latency and VALU: about 30
 // instructions, two of them transcendental, for each of the 7.2 M mix values.
 constexpr int kTileTok = 16;
 constexpr int kLowBlocks = 3;                 // 16-row blocks of projection rows per block
