@@ -329,12 +329,12 @@ hipError_t launch_grouped(int epi, const GroupedLaunch& p, uint32_t max_tiles, h
 // The 16-row tile kernels of small calls (see k_rows); false when K is above
 // their LDS bound.
 constexpr int kRowsTile = 16;
+bool rows_supported(uint32_t k_dim);
 // The down GEMM's staged-weight instances (and so its tall tiles) take this K.
 bool down_tall_supported(uint32_t k_dim);
 // K of half a chunk over, and the column slices of the chunked down GEMM.
 bool down_half_tail(uint32_t k_dim);
 uint32_t down_slices(uint32_t n_dim);
-bool rows_supported(uint32_t k_dim);
 hipError_t launch_rows(int epi, const GroupedLaunch& p, uint32_t max_tiles, hipStream_t stream);
 // The down GEMM over tiles of up to kGroupedRowsDown rows with whole A rows in
 // LDS (k_down_rows).
